@@ -399,7 +399,8 @@ int mpq_awq_search(const float* W, int64_t rows, int64_t n, const float* H, cons
  * (H = 2/m sum x x^T, mpq/adapters/gptqmodel.py:39) and QUIP#'s Hessian hooks
  * (mpq/quip_generic.py:823-921: sum x x^T and sum x, finalised as H/ct - mu mu^T).
  *   X: T x n activations (ldx >= n, ldx % 4 == 0), fp32 (x_bf16 = 0) or bf16 (x_bf16 = 1);
- *   n % 128 == 0; H: n x n fp32 (ldh).  fp32 MFMA SYRK (tiles on/above the diagonal).
+ *   n % 128 == 0; H: n x n fp32 (ldh).  SYRK on the bf16 matrix cores (tiles
+ *   on/above the diagonal; fp32 X as three exact bf16 planes, fp32 accuracy).
  */
 int mpq_hessian_accumulate(const void* X, int x_bf16, int64_t T, int64_t n, int64_t ldx, float alpha,
                            float beta, float* H, int64_t ldh, float* colsum, mpq_stream_t stream);

@@ -6,173 +6,242 @@
 // (mpq/quip_generic.py:823-921, H / ct - mu mu^T).  Both are one symmetric rank-T update per
 // batch of T activations X (T x n, fp32 or bf16).
 //
-// SYRK on fp32 MFMA (v_mfma_f32_32x32x2_f32): 128 x 64 output tiles, only tiles on or above the
-// diagonal do work; each computed element is written to (m, n) and mirrored to (n, m), so H stays
-// exactly symmetric.  A = X^T needs no transpose in LDS: a K slab of X^T (128 columns of X, 16
-// rows) is loaded along m with float4 reads and stored as [k][m], the layout the MFMA operand
-// reads use.  Two K slabs of global loads are in flight (register sets R0/R1).
+// SYRK on the bf16 matrix cores (v_mfma_f32_32x32x16_bf16, fp32 accumulation).  bf16 activations are
+// their own plane, and every product of two bf16 values is exact in the fp32 accumulator.  fp32
+// activations are split exactly into three bf16 planes (x6_split.h) and the six plane products of
+// order >= 2^-16 |a||b| are kept, the accuracy of an fp32 product.  The accumulator is rounded once per
+// 16 tokens, where v_mfma_f32_32x32x2_f32 rounds once per 2.
 #include <hip/hip_bf16.h>
 
+#include <type_traits>
+
 #include "common.h"
+#include "x6_split.h"
 
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-constexpr int BM = 128, BN = 64, WM = 64, WN = 32, BK = 16;
 constexpr int kThreads = 256;
 
-template <bool kBf16>
-__device__ __forceinline__ float4 load4(const void* base, int64_t idx, bool ok) {
-  if (!ok) return make_float4(0.f, 0.f, 0.f, 0.f);
-  if constexpr (kBf16) {
-    const __hip_bfloat16* p = static_cast<const __hip_bfloat16*>(base) + idx;
-    const uint2 raw = *reinterpret_cast<const uint2*>(p);
-    return make_float4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xffff0000u),
-                       __uint_as_float(raw.y << 16), __uint_as_float(raw.y & 0xffff0000u));
-  } else {
-    return *reinterpret_cast<const float4*>(static_cast<const float*>(base) + idx);
-  }
+__device__ __noinline__ float column_dot(const float* __restrict__ X, int64_t T, int64_t ldx, int64_t i, int64_t j) {
+  float acc = 0.f;
+  for (int64_t t = 0; t < T && !isnan(acc); ++t) acc = fmaf(X[t * ldx + i], X[t * ldx + j], acc);
+  return acc;
 }
 
-template <bool kBf16>
-__global__ __launch_bounds__(kThreads) void syrk_kernel(const void* __restrict__ X, int64_t T, int64_t n,
+// H tile (TS x TS, on or above the diagonal) = beta H + alpha X^T X, mirrored to the transposed tile,
+// so H stays exactly symmetric.  Four waves of TS/2 x TS/2.
+//
+// Both operands are column panels of X (token-major), but an MFMA operand wants 8 consecutive tokens
+// of one column per lane.  A thread loads R tokens x 4 columns, transposes them in registers and writes
+// one 2R-byte piece per column to LDS: [plane][8-token group][slot], 16 bytes per slot, with column m at
+// slot (m % 4) * TS/4 + m / 4, so a wave's writes and its fragment reads are both contiguous.  Two LDS
+// buffers, D slabs of loads in flight in registers, one barrier per slab.
+//
+// Bound: bf16, the LDS fragment reads (1 KB per MFMA and wave with 64 x 64 wave tiles: the LDS rate);
+// fp32, the matrix cores (six products per fragment pair).  4096 columns x 16384 tokens
+// bf16: 4660 -> 575 us (478 TFLOP/s of n^2 T); 14336 x 8192 bf16: 18.7 -> 2.7 ms (616 TFLOP/s); 2048 x 3001
+// fp32: 221 -> 135 us, both against one fp32 MFMA kernel for either type.
+template <bool kBf16, int TS>
+__global__ __launch_bounds__(kThreads, 2) void syrk_kernel(const void* __restrict__ X, int64_t T, int64_t n,
                                                         int64_t ldx, float alpha, float beta,
                                                         float* __restrict__ H, int64_t ldh) {
-  constexpr int WAVES_N = BN / WN;
-  constexpr int MI = WM / 32, NI = WN / 32;
-  constexpr int A_F4 = BM * BK / 4 / kThreads;  // 2
-  constexpr int B_F4 = BN * BK / 4 / kThreads;  // 1
-  __shared__ float As[2][BK][BM + 4];
-  __shared__ float Bs[2][BK][BN + 4];
+  constexpr int NP = kBf16 ? 1 : 3;
+  constexpr int NQ = TS / 4;                    // column quads of a tile
+  constexpr int R = kBf16 && TS == 128 ? 8 : 4;  // tokens per thread and slab
+  constexpr int KS = R * 128 / NQ;              // tokens per slab: 32 (16: fp32, TS = 128)
+  constexpr int NB = TS / 64;                   // 32 x 32 blocks per wave and dimension
+  constexpr int D = !kBf16 && TS == 128 ? 2 : 4;  // slabs of loads in flight (even)
+  __shared__ uint4 As[2][NP][KS / 8][TS];
+  __shared__ uint4 Bs[2][NP][KS / 8][TS];
 
-  const int64_t m0 = (int64_t)blockIdx.y * BM;
-  const int64_t n0 = (int64_t)blockIdx.x * BN;
-  if (n0 + BN <= m0) return;  // strictly below the diagonal: mirrored from its transpose tile
+  // upper-triangular tile index -> (ti, tj), ti <= tj: tj (tj + 1) / 2 tiles precede column tj
+  const int t = (int)blockIdx.x;
+  int tj = (int)((sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);
+  while ((tj + 1) * (tj + 2) / 2 <= t) ++tj;
+  while (tj * (tj + 1) / 2 > t) --tj;
+  const int ti = t - tj * (tj + 1) / 2;
+  const int64_t m0 = (int64_t)ti * TS, n0 = (int64_t)tj * TS;
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm0 = (wave / WAVES_N) * WM;
-  const int wn0 = (wave % WAVES_N) * WN;
-  const int64_t nslab = (T + BK - 1) / BK;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int op = tid >> 7, c = (tid & 127) % NQ, kg = (tid & 127) / NQ;
+  typedef typename std::conditional<kBf16, uint2, float4>::type Quad;  // four columns of one token
+  const char* mine = static_cast<const char*>(X) + (kg * R * ldx + (op ? n0 : m0) + 4 * c) * (kBf16 ? 2 : 4);
+  const int64_t nslab = (T + KS - 1) / KS;
 
-  float4 ra0[A_F4], rb0[B_F4], ra1[A_F4], rb1[B_F4];
-  // A(m, k) = X[k][m0 + m]: thread t loads 4 consecutive m of row k
-  auto gload = [&](float4 (&ra)[A_F4], float4 (&rb)[B_F4], int64_t s) {
+  Quad r[D][R];
+  auto gload = [&](int64_t s, int set) {
+    const int64_t left = T - s * KS - kg * R;  // tokens from this thread's first one on
 #pragma unroll
-    for (int i = 0; i < A_F4; ++i) {
-      const int t = tid + i * kThreads;
-      const int k = t / (BM / 4);
-      const int mq = (t % (BM / 4)) * 4;
-      const int64_t gk = s * BK + k;
-      ra[i] = load4<kBf16>(X, gk * ldx + m0 + mq, gk < T);
-    }
-#pragma unroll
-    for (int i = 0; i < B_F4; ++i) {
-      const int t = tid + i * kThreads;
-      const int k = t / (BN / 4);
-      const int nq = (t % (BN / 4)) * 4;
-      const int64_t gk = s * BK + k;
-      rb[i] = load4<kBf16>(X, gk * ldx + n0 + nq, gk < T);
+    for (int e = 0; e < R; ++e) {
+      r[set][e] = Quad{};
+      if (e < left) r[set][e] = *reinterpret_cast<const Quad*>(mine + (s * KS + e) * ldx * (kBf16 ? 2 : 4));
     }
   };
-  auto lstore = [&](const float4 (&ra)[A_F4], const float4 (&rb)[B_F4], int buf) {
-#pragma unroll
-    for (int i = 0; i < A_F4; ++i) {
-      const int t = tid + i * kThreads;
-      *reinterpret_cast<float4*>(&As[buf][t / (BM / 4)][(t % (BM / 4)) * 4]) = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < B_F4; ++i) {
-      const int t = tid + i * kThreads;
-      *reinterpret_cast<float4*>(&Bs[buf][t / (BN / 4)][(t % (BN / 4)) * 4]) = rb[i];
-    }
+  auto put = [&](int buf, int pl, int j, const uint32_t (&w)[R / 2]) {
+    uint4* slot = op ? &Bs[buf][pl][kg * R / 8][j * NQ + c] : &As[buf][pl][kg * R / 8][j * NQ + c];
+    if constexpr (R == 8)
+      *slot = make_uint4(w[0], w[1], w[2], w[3]);
+    else
+      reinterpret_cast<uint2*>(slot)[kg & 1] = make_uint2(w[0], w[1]);
   };
-
-  floatx16 acc[MI][NI];
+  auto lstore = [&](int set, int buf) {
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+    for (int j = 0; j < 4; ++j) {
+      uint32_t w[NP][R / 2];
 #pragma unroll
-    for (int j = 0; j < NI; ++j)
+      for (int d = 0; d < R / 2; ++d) {
+        if constexpr (kBf16) {
+          const uint2 p = r[set][2 * d], q = r[set][2 * d + 1];
+          const uint32_t lo = j < 2 ? p.x : p.y, hi = j < 2 ? q.x : q.y;
+          w[0][d] = __builtin_amdgcn_perm(hi, lo, j & 1 ? 0x07060302u : 0x05040100u);
+        } else {
+          const float4 a = r[set][2 * d], b = r[set][2 * d + 1];
+          const float x = j == 0 ? a.x : j == 1 ? a.y : j == 2 ? a.z : a.w;
+          const float y = j == 0 ? b.x : j == 1 ? b.y : j == 2 ? b.z : b.w;
+          mpq::split3(x, y, w[0][d], w[1][d], w[2][d]);
+        }
+      }
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-  const int kl = lane >> 5;
-  const int ml = lane & 31;
-  auto compute = [&](int buf) {
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 2) {
-      float a[MI], b[NI];
-#pragma unroll
-      for (int i = 0; i < MI; ++i) a[i] = As[buf][kk + kl][wm0 + i * 32 + ml];
-#pragma unroll
-      for (int j = 0; j < NI; ++j) b[j] = Bs[buf][kk + kl][wn0 + j * 32 + ml];
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
+      for (int pl = 0; pl < NP; ++pl) put(buf, pl, j, w[pl]);
     }
   };
 
-  gload(ra0, rb0, 0);
-  if (nslab > 1) gload(ra1, rb1, 1);
-  lstore(ra0, rb0, 0);
-  __syncthreads();
-  // Pairs of slabs with no exit inside the body (an exit between the halves makes the compiler
-  // copy every accumulator through VGPRs each iteration, draining the MFMA pipeline); an odd last
-  // slab, already in LDS buffer 0, is computed after the loop.
-  int64_t s = 0;
-  for (; s + 1 < nslab; s += 2) {
-    if (s + 2 < nslab) gload(ra0, rb0, s + 2);
-    compute(0);
-    lstore(ra1, rb1, 1);
-    __syncthreads();
-    if (s + 3 < nslab) gload(ra1, rb1, s + 3);
-    compute(1);
-    if (s + 2 < nslab) lstore(ra0, rb0, 0);
-    __syncthreads();
-  }
-  if (s < nslab) compute(0);
-
-  // epilogue: elements on or above the diagonal, value written to (m, n) and (n, m)
-  const int col = lane & 31;
-  const int rbase = (lane >> 5) * 4;
+  // the small plane products have accumulators of their own: every sum into the large one costs half an
+  // ulp of it whatever is added (one accumulator for all six: relative error 3.0e-6 instead of 6.5e-7 at
+  // 4096 x 16384; fp32 MFMA 2.0e-6)
+  floatx16 acc[NB][NB], low[NP == 3 ? NB : 1][NB];
 #pragma unroll
-  for (int i = 0; i < MI; ++i) {
+  for (int i = 0; i < NB; ++i)
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const int64_t gn = n0 + wn0 + j * 32 + col;
+    for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int64_t gm = m0 + wm0 + i * 32 + (v >> 2) * 8 + rbase + (v & 3);
+        acc[i][j][v] = 0.f;
+        if constexpr (NP == 3) low[i][j][v] = 0.f;
+      }
+  const int sm = (wave >> 1) * (TS / 2) + (lane & 31), sn = (wave & 1) * (TS / 2) + (lane & 31);
+  auto compute = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < KS / 16; ++k) {
+      bf16x8 a[NP][NB], b[NP][NB];
+#pragma unroll
+      for (int pl = 0; pl < NP; ++pl)
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+          a[pl][i] = __builtin_bit_cast(bf16x8, As[buf][pl][2 * k + (lane >> 5)][sm + 32 * i]);
+          b[pl][i] = __builtin_bit_cast(bf16x8, Bs[buf][pl][2 * k + (lane >> 5)][sn + 32 * i]);
+        }
+      if constexpr (NP == 3) {  // smallest terms first
+        constexpr int pa[5] = {2, 1, 0, 1, 0};
+        constexpr int pb[5] = {0, 1, 2, 0, 1};
+#pragma unroll
+        for (int q = 0; q < 5; ++q)
+#pragma unroll
+          for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+              low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[q]][i], b[pb[q]][j], low[i][j], 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[0][j], acc[i][j], 0, 0, 0);
+    }
+  };
+
+  // Slab s is in LDS buffer s & 1, slabs s + 1 .. s + D - 1 are in flight in the register sets s % D.
+  // Rounds of D slabs with no exit inside; the slabs past the last token load nothing and multiply zeros.
+  // The barrier waits for this wave's LDS accesses only: __syncthreads would also wait for the loads in
+  // flight.
+  auto barrier = []() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+#pragma unroll
+  for (int u = 0; u < D; ++u) gload(u, u);
+  lstore(0, 0);
+  barrier();
+  for (int64_t s0 = 0; s0 < nslab; s0 += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      gload(s0 + u + D, u);
+      compute(u & 1);
+      lstore((u + 1) % D, (u + 1) & 1);
+      barrier();
+    }
+  }
+
+  // slot s of an operand is column 4 (s % NQ) + s / NQ of its panel; elements on or above the diagonal
+  // are written to (m, n) and (n, m)
+  auto col_of = [](int s) { return 4 * (s % NQ) + s / NQ; };
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int64_t gn = n0 + col_of(sn + 32 * j);
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int64_t gm = m0 + col_of((wave >> 1) * (TS / 2) + 32 * i + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3));
         if (gn < gm) continue;
         float* dst = H + gm * ldh + gn;
-        const float val = beta == 0.f ? alpha * acc[i][j][v] : alpha * acc[i][j][v] + beta * *dst;
+        float sum = acc[i][j][v];
+        if constexpr (NP == 3) sum += low[i][j][v];
+        // the planes of an infinity (or of a value that rounds to one in bf16) are not finite: such an
+        // entry is summed again from the activations, so it overflows as an fp32 product does
+        if (!kBf16 && isnan(sum)) sum = column_dot(static_cast<const float*>(X), T, ldx, gm, gn);
+        const float val = beta == 0.f ? alpha * sum : alpha * sum + beta * *dst;
         *dst = val;
         if (gn != gm) H[gn * ldh + gm] = val;
       }
     }
-  }
 }
 
-// colsum[j] += sum_t X[t][j] (fixed order: per-thread column, rows in order).
+// colsum[j] += sum_t X[t][j], in a fixed order: a work-group owns 16 columns, thread (g, j) adds the
+// tokens g, g + 64, ... of column j, and the 64 sums of a column are added pairwise in LDS.  One work-group
+// per 16 columns with 64 token streams keeps enough loads in flight (2048 columns x 3001 tokens fp32:
+// 10 us; one thread per column took 691 us, a chain of 3001 loads in 8 work-groups).
 template <bool kBf16>
-__global__ __launch_bounds__(256) void colsum_kernel(const void* __restrict__ X, int64_t T, int64_t n, int64_t ldx,
-                                                     float* __restrict__ colsum) {
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
+__global__ __launch_bounds__(1024) void colsum_kernel(const void* __restrict__ X, int64_t T, int64_t n, int64_t ldx,
+                                                      float* __restrict__ colsum) {
+  __shared__ float red[64][17];
+  const int j = threadIdx.x & 15, g = threadIdx.x >> 4;
+  const int64_t col = (int64_t)blockIdx.x * 16 + j;  // n % 128 == 0: every column exists
   float acc = 0.f;
-  for (int64_t t = 0; t < T; ++t) {
-    float v;
+#pragma unroll 4
+  for (int64_t t = g; t < T; t += 64) {
     if constexpr (kBf16) {
-      v = __bfloat162float(static_cast<const __hip_bfloat16*>(X)[t * ldx + j]);
+      acc += __bfloat162float(static_cast<const __hip_bfloat16*>(X)[t * ldx + col]);
     } else {
-      v = static_cast<const float*>(X)[t * ldx + j];
+      acc += static_cast<const float*>(X)[t * ldx + col];
     }
-    acc += v;
   }
-  colsum[j] += acc;
+  red[g][j] = acc;
+  __syncthreads();
+  for (int w = 32; w > 0; w >>= 1) {
+    if (g < w) red[g][j] += red[g + w][j];
+    __syncthreads();
+  }
+  if (g == 0) colsum[col] += red[0][j];
+}
+
+template <bool kBf16>
+void launch(const void* X, int64_t T, int64_t n, int64_t ldx, float alpha, float beta, float* H, int64_t ldh,
+            float* colsum, hipStream_t stream) {
+  // 128 x 128 tiles read half as much LDS per product, but well below one tile per CU the chip idles:
+  // there 64 x 64 tiles (four times as many).  8192 tokens, 128 / 64 tiles, us: n = 1024 bf16 143 / 96,
+  // fp32 460 / 195; 2304 (171 tiles) 152 / 132, 462 / 366; 2816 (253 tiles) 160 / 167, 478 / 521;
+  // 4096 271 / 369, 1092 / 1058; 8192 935 / 1337, 3365 / 4233.
+  const int64_t nt = n / 128, tiles = nt * (nt + 1) / 2;
+  if (tiles >= 200) {
+    hipLaunchKernelGGL((syrk_kernel<kBf16, 128>), dim3((unsigned)tiles), dim3(kThreads), 0, stream, X, T, n, ldx,
+                       alpha, beta, H, ldh);
+  } else {
+    hipLaunchKernelGGL((syrk_kernel<kBf16, 64>), dim3((unsigned)(nt * (2 * nt + 1))), dim3(kThreads), 0, stream, X, T,
+                       n, ldx, alpha, beta, H, ldh);
+  }
+  if (colsum)
+    hipLaunchKernelGGL(colsum_kernel<kBf16>, dim3((unsigned)(n / 16)), dim3(1024), 0, stream, X, T, n, ldx, colsum);
 }
 
 }  // namespace
@@ -187,18 +256,8 @@ extern "C" int mpq_hessian_accumulate(const void* X, int x_bf16, int64_t T, int6
   MPQ_CHECK_ARG(T == 0 || (reinterpret_cast<uintptr_t>(X) & (x_bf16 ? 7u : 15u)) == 0,
                 "mpq_hessian_accumulate: X must be 16-byte (fp32) / 8-byte (bf16) aligned");
   MPQ_CHECK_ARG(n / 64 <= 65535, "mpq_hessian_accumulate: n too large");
-  const dim3 grid((unsigned)(n / BN), (unsigned)(n / BM));
-  if (x_bf16) {
-    hipLaunchKernelGGL(syrk_kernel<true>, grid, dim3(kThreads), 0, stream, X, T, n, ldx, alpha, beta, H, ldh);
-    if (colsum)
-      hipLaunchKernelGGL(colsum_kernel<true>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, X, T, n, ldx,
-                         colsum);
-  } else {
-    hipLaunchKernelGGL(syrk_kernel<false>, grid, dim3(kThreads), 0, stream, X, T, n, ldx, alpha, beta, H, ldh);
-    if (colsum)
-      hipLaunchKernelGGL(colsum_kernel<false>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, X, T, n,
-                         ldx, colsum);
-  }
+  if (x_bf16) launch<true>(X, T, n, ldx, alpha, beta, H, ldh, colsum, stream);
+  else launch<false>(X, T, n, ldx, alpha, beta, H, ldh, colsum, stream);
   MPQ_LAUNCH_CHECK();
   return kOk;
 }

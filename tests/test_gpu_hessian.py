@@ -1,4 +1,4 @@
-"""GPU: Hessian accumulation (mpq_hessian_accumulate, fp32 MFMA SYRK) against fp64 products, and
+"""GPU: Hessian accumulation (mpq_hessian_accumulate, bf16 MFMA SYRK) against fp64 products, and
 the GPTQ / QUIP# accumulation conventions (mpq_amd/hessian.py) against fp64 restatements."""
 import math
 
@@ -76,3 +76,40 @@ def test_quip_convention(gpu):
 def test_rejects_bad_width(gpu):
     with pytest.raises(ValueError):
         hessian.accumulate(torch.zeros(100, 100, device=gpu), torch.zeros(10, 100, device=gpu))
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("T,n", [(1, 128), (31, 128), (33, 384), (127, 640), (129, 2432), (100, 2560)])
+def test_syrk_slab_and_tile_edges(gpu, T, n, bf16):
+    """Partial token slabs, the 64 x 64 tiles (below 200 tiles of 128 x 128: n <= 2432) and the 128 x 128
+    tiles, and the column sums.  Each entry sums T products exact to 2^-22 relative in fp32: its error is
+    at most (2^-22 + (T + 2) 2^-24) sum |x_i x_j|."""
+    g = torch.Generator().manual_seed(7 * T + n)
+    X = torch.randn(T, n, generator=g) * torch.exp(torch.randn(n, generator=g))
+    X = X.to(torch.bfloat16) if bf16 else X
+    H = torch.zeros(n, n, device=gpu)
+    cs = torch.ones(n, device=gpu)
+    hessian.accumulate(H, X.to(gpu), colsum=cs)
+    Xd = X.double().to(gpu)
+    bound = (2.0 ** -22 + (T + 2) * 2.0 ** -24) * (Xd.abs().T @ Xd.abs())
+    assert bool(((H.double() - Xd.T @ Xd).abs() <= bound).all())
+    assert torch.equal(H, H.T)
+    assert bool(((cs.double() - 1 - Xd.sum(0)).abs() <= (T + 2) * 2.0 ** -24 * (1 + Xd.abs().sum(0))).all())
+
+
+@pytest.mark.parametrize("n", [256, 2560])
+def test_syrk_non_finite_activations(gpu, n):
+    """Infinities, NaN and values that round to an infinity in bf16 act as in fp32 products."""
+    g = torch.Generator().manual_seed(n)
+    X = torch.randn(40, n, generator=g)
+    X[5, 7], X[9, 100], X[3, 50] = float("inf"), float("nan"), 3.4e38
+    X[3, 7] = 0.5  # 3.4e38 X[3, 7] must not overflow before the infinity of column 7 is added (fp32 would give NaN)
+    H = torch.zeros(n, n, device=gpu)
+    hessian.accumulate(H, X.to(gpu))
+    H = H.cpu()
+    ref = X.double().T @ X.double()
+    ref = torch.where(ref.abs() > 3.4028235e38, ref.sign() * float("inf"), ref)
+    assert torch.equal(torch.isnan(H), torch.isnan(ref))
+    assert torch.equal(torch.isinf(H), torch.isinf(ref)) and torch.equal(H[torch.isinf(H)], ref[torch.isinf(ref)].float())
+    ok = torch.isfinite(H)
+    assert float((H[ok].double() - ref[ok]).abs().max() / 3.4e38) < 1e-6
