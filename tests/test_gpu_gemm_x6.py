@@ -118,3 +118,71 @@ def test_gemm_x6_splitk_partials_sum_to_the_product(gpu):
     for s in (0, splits - 1):
         ref = A[:, s * ks:(s + 1) * ks].double() @ B[s * ks:(s + 1) * ks].double()
         assert float((P[s].cpu().double() - ref).abs().max()) <= 2e-6 * float(ref.abs().max())
+
+
+def _pair_bound(A, B):
+    """Error bound of one product from the f16 pairs.  Each operand is held to 2^-23 relative, or absolutely
+    to 2^-39 of the largest of its row's 1024 columns (A: that one is scaled to 2^14 .. 2^15, and the low
+    plane's last subnormal bit is 2^-24) and 2^-37 of its column's largest (B: scaled to at least 2^12); the
+    dropped low x low product is 2^-22 relative.  The fp32 roundings of the sums stay below what is
+    left of 2^-20 relative for the sizes tested."""
+    M, K = A.shape
+    amax = torch.zeros_like(A)
+    for c in range(0, K, 1024):
+        amax[:, c:c + 1024] = A[:, c:c + 1024].abs().amax(1, keepdim=True)
+    bmax = B.abs().amax(0, keepdim=True).expand_as(B)
+    return 2.0 ** -20 * (A.abs() @ B.abs()) + 2.0 ** -39 * (amax @ B.abs()) + 2.0 ** -37 * (A.abs() @ bmax)
+
+
+@pytest.mark.parametrize("M,N,K,splits", [
+    (3, 128, 32, 1), (128, 128, 1024, 1), (129, 256, 1056, 1), (128, 128, 2112, 3), (100, 128, 96, 1),
+    (128, 128, 17 * 1024, 1),    # more chunks of A's scales than a work-group keeps in LDS
+    (65, 128, 17 * 1024 + 32, 1),  # the same with a ragged slab count
+    (128, 256, 3584, 1), (64, 128, 4096, 8)])
+def test_pair_product_slices_and_chunks(gpu, M, N, K, splits):
+    """Slab counts that are not multiples of the ring's four stages, one and many 1024-column chunks."""
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g).double().to(gpu)
+    B = torch.randn(K, N, generator=g).double().to(gpu)
+    Ap, Bp = ops.gemm_x6_pack_a(A.float()), ops.gemm_x6_pack_b(B.float())
+    P, _ = ops.gemm_x6_splitk(Ap, Bp, M, N, K, splits=splits)
+    assert bool(((P.double().sum(0) - A @ B).abs() <= _pair_bound(A, B)).all())
+
+
+def test_pair_product_scales_follow_the_data(gpu):
+    """Chunks of A and columns of B over 60 orders of magnitude: zero slabs first, columns that grow and
+    shrink along K, values far below their group's largest (subnormal planes), zero rows and columns."""
+    M, N, K = 128, 256, 4096
+    g = torch.Generator().manual_seed(77)
+    A = torch.randn(M, K, generator=g).double()
+    B = torch.randn(K, N, generator=g).double()
+    A[:32] *= 1e-30
+    A[32:64, 1024:2048] *= 1e12   # chunk maxima 1, 1e12, 1, 1
+    A[64:96, 2048:] *= 1e-20
+    A[96] = 0.0
+    k = torch.arange(K, dtype=torch.float64).view(-1, 1)
+    B[:, :32] *= torch.exp2(k / 64)          # grows by 2^64
+    B[:, 32:64] *= torch.exp2(-k / 64)       # shrinks by 2^64
+    B[:2000, 64:96] = 0.0                    # zero until a late slab
+    B[:, 96:128] *= 1e20  # times 1e12 of A, still an fp32 number
+    B[:, 128:160] *= 1e-7
+    B[5, 128:160] = 1.0                      # one value 2^23 above the others, against a zero of A
+    A[:16, 5] = 0.0
+    B[:, 200] = 0.0
+    A, B = A.float().double().to(gpu), B.float().double().to(gpu)
+    C = ops.gemm_x6(A.float(), ops.gemm_x6_pack_b(B.float()), N).double()
+    err, bound = (C - A @ B).abs(), _pair_bound(A, B)
+    assert bool((err <= bound).all()), float((err / bound).nan_to_num(0).max())
+    assert float(C[96].abs().max()) == 0.0 and float(C[:, 200].abs().max()) == 0.0
+
+
+def test_pair_product_non_finite_stays_in_its_row_and_column(gpu):
+    M, N, K = 40, 128, 2048
+    g = torch.Generator().manual_seed(5)
+    A, B = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g)
+    C0 = ops.gemm_x6(A.to(gpu), ops.gemm_x6_pack_b(B.to(gpu)), N).cpu()
+    A[3, 1500], A[7, 2], B[900, 11] = float("inf"), float("nan"), float("-inf")
+    C = ops.gemm_x6(A.to(gpu), ops.gemm_x6_pack_b(B.to(gpu)), N).cpu()
+    bad = torch.zeros(M, N, dtype=torch.bool)
+    bad[3], bad[7], bad[:, 11] = True, True, True
+    assert not bool(torch.isfinite(C[bad]).any()) and torch.equal(C[~bad], C0[~bad])
