@@ -473,7 +473,7 @@ int uniform_cd_polish(int64_t rows, int64_t n, int maxq, int64_t block_rows, int
       Wc = scratch;
     }
     MPQ_HIP_TRY(product_splits(Wc, Vs, false, rows, n, P, pl.splits, pl.bn, stream));
-    MPQ_HIP_TRY(splitk_reduce(P, pl.splits, rows, n, Yu, n, 1.f, 0.f, stream));
+    MPQ_HIP_TRY(splitk_reduce(P, pl.splits, sstride, rows, n, Yu, n, 1.f, 0.f, stream));
   }
   // x (given, or from the codes); residual and its norm (= error before the polish)
   if (x_in) {
@@ -499,10 +499,10 @@ int uniform_cd_polish(int64_t rows, int64_t n, int maxq, int64_t block_rows, int
   if (x6) {
     MPQ_HIP_TRY(x6_pack_a(scratch, n, rows, n, Ap, stream, S));
     MPQ_HIP_TRY(x6_gemm_partials(Ap, packed + n * n, rows, n, n, P, n, sstride, pl.splits_x6, stream));
-    MPQ_HIP_TRY(splitk_reduce(P, pl.splits_x6, rows, n, rhs, n, 1.f, 0.f, stream));
+    MPQ_HIP_TRY(splitk_reduce(P, pl.splits_x6, sstride, rows, n, rhs, n, 1.f, 0.f, stream));
   } else {
     MPQ_HIP_TRY(product_splits(scratch, Vs, true, rows, n, P, pl.splits, pl.bn, stream));
-    MPQ_HIP_TRY(splitk_reduce(P, pl.splits, rows, n, rhs, n, 1.f, 0.f, stream));
+    MPQ_HIP_TRY(splitk_reduce(P, pl.splits, sstride, rows, n, rhs, n, 1.f, 0.f, stream));
   }
   MPQ_HIP_TRY(row_sqnorm(Vs, n, n, 1e-12f, diag, stream));
   hipLaunchKernelGGL(recip_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, n, diag, diag_inv);

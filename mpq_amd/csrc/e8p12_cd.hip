@@ -755,7 +755,7 @@ extern "C" int mpq_e8p12_cd_polish(int64_t rows, int64_t n, int64_t block_rows, 
     MPQ_HIP_TRY(hipMemcpyAsync(Yu, Yu_in, rows * n * 4, hipMemcpyDeviceToDevice, stream));
   } else {
     MPQ_HIP_TRY(product_splits(W, Vs, false, rows, n, P, pl.splits, pl.bn, stream));
-    MPQ_HIP_TRY(splitk_reduce(P, pl.splits, rows, n, Yu, n, 1.f, 0.f, stream));
+    MPQ_HIP_TRY(splitk_reduce(P, pl.splits, sstride, rows, n, Yu, n, 1.f, 0.f, stream));
   }
   MPQ_HIP_TRY(hipMemcpyAsync(x_out, x_in, rows * n * 4, hipMemcpyDeviceToDevice, stream));
   MPQ_HIP_TRY(hipMemcpyAsync(idx_out, idx_in, rows * nb * 8, hipMemcpyDeviceToDevice, stream));
@@ -769,7 +769,7 @@ extern "C" int mpq_e8p12_cd_polish(int64_t rows, int64_t n, int64_t block_rows, 
   MPQ_HIP_TRY(hipMemcpyAsync(res, err_b, rows * 4, hipMemcpyDeviceToDevice, stream));
   MPQ_HIP_TRY(hipMemsetAsync(acc, 0, rows * 4, stream));
   MPQ_HIP_TRY(product_splits(resid, Vs, true, rows, n, P, pl.splits, pl.bn, stream));
-  MPQ_HIP_TRY(splitk_reduce(P, pl.splits, rows, n, rhs, n, 1.f, 0.f, stream));
+  MPQ_HIP_TRY(splitk_reduce(P, pl.splits, sstride, rows, n, rhs, n, 1.f, 0.f, stream));
 
   const int64_t nsteps = (max_blocks > 0 && max_blocks < nb) ? max_blocks : nb;
   const int64_t row_tiles = pl.nrb * tiles_per_rb;

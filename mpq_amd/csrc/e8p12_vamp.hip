@@ -198,7 +198,7 @@ extern "C" int mpq_e8p12_vamp_solve_ex(int64_t rows, int64_t n, const float* Wr,
 
   // ---- setup: Yu, gamma1, obs warm start
   MPQ_HIP_TRY(prod(Wr, Vs, false, 2));
-  MPQ_HIP_TRY(splitk_reduce(P, nsplit, rows, n, Yu, n, 1.f, 0.f, stream));
+  MPQ_HIP_TRY(splitk_reduce(P, nsplit, sstride, rows, n, Yu, n, 1.f, 0.f, stream));
   MPQ_HIP_TRY(prod(hat_init, Vs, false, 2));
   hipLaunchKernelGGL(err_epi_kernel, eg, eb, 0, stream, n, P, nsplit, sstride, Yu, part, nullptr);
   hipLaunchKernelGGL(rows_err_kernel, dim3(1), eb, 0, stream, rows, nchunks, part, errrow, status, nullptr, 0u);

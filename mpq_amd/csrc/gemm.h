@@ -39,9 +39,9 @@ int choose_splits(int64_t M, int64_t N, int64_t K, int64_t workspace_floats, int
 // p.split_stride apart (mode kGemmPartials), or one slice with mode kGemmAxpby.
 hipError_t gemm_partials(GemmParams p, int splits, int bn, hipStream_t stream);
 
-// C = alpha * sum_s P[s] + beta * C (fixed split order).
-hipError_t splitk_reduce(const float* P, int splits, int64_t M, int64_t N, float* C, int64_t ldc,
-                         float alpha, float beta, hipStream_t stream);
+// C = alpha * sum_s P[s] + beta * C (fixed split order); P[s] at P + s * split_stride.
+hipError_t splitk_reduce(const float* P, int splits, int64_t split_stride, int64_t M, int64_t N, float* C,
+                         int64_t ldc, float alpha, float beta, hipStream_t stream);
 
 // Full product with the automatic split choice; `workspace` may be null (1 split).
 hipError_t gemm(const float* A, int64_t lda, const float* B, int64_t ldb, bool trans_b,

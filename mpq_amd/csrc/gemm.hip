@@ -767,13 +767,13 @@ hipError_t gemm_partials(GemmParams p, int splits, int bn, hipStream_t stream) {
   return launch_cfg<128, 64, 64, 32>(p, grid, stream);
 }
 
-hipError_t splitk_reduce(const float* P, int splits, int64_t M, int64_t N, float* C, int64_t ldc,
-                         float alpha, float beta, hipStream_t stream) {
+hipError_t splitk_reduce(const float* P, int splits, int64_t split_stride, int64_t M, int64_t N, float* C,
+                         int64_t ldc, float alpha, float beta, hipStream_t stream) {
   const int64_t total = M * N;
   int64_t blocks = (total + 255) / 256;
   if (blocks > 8192) blocks = 8192;
   hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, P, splits,
-                     M * N, M, N, C, ldc, alpha, beta);
+                     split_stride, M, N, C, ldc, alpha, beta);
   return hipGetLastError();
 }
 
@@ -870,7 +870,7 @@ hipError_t gemm(const float* A, int64_t lda, const float* B, int64_t ldb, bool t
   p.C = workspace; p.ldc = N; p.split_stride = M * N;
   hipError_t e = gemm_partials(p, splits, bn, stream);
   if (e != hipSuccess) return e;
-  return splitk_reduce(workspace, splits, M, N, C, ldc, alpha, beta, stream);
+  return splitk_reduce(workspace, splits, M * N, M, N, C, ldc, alpha, beta, stream);
 }
 
 }  // namespace mpq
@@ -949,7 +949,7 @@ extern "C" int mpq_gemm_x6(int64_t M, int64_t N, int64_t K, const float* A, int6
   float* P = reinterpret_cast<float*>(ws + (mpq::x6_packed_a_bytes(M, K) + 255) / 256 * 256);
   MPQ_HIP_TRY(mpq::x6_pack_a(A, lda, M, K, ws, stream));
   MPQ_HIP_TRY(mpq::x6_gemm_partials(ws, B_packed, M, N, K, P, N, M * N, splits, stream));
-  MPQ_HIP_TRY(mpq::splitk_reduce(P, splits, M, N, C, ldc, 1.f, 0.f, stream));
+  MPQ_HIP_TRY(mpq::splitk_reduce(P, splits, M * N, M, N, C, ldc, 1.f, 0.f, stream));
   return mpq::kOk;
 }
 

@@ -425,7 +425,7 @@ int uniform_vamp_solve(const UniformProblem& pr, const float* Vs, const MpqUnifo
       Wc = w.r1;
     }
     MPQ_HIP_TRY(product(w, Wc, Vs, false, kOpVs, rows, n, stream));
-    MPQ_HIP_TRY(splitk_reduce(w.P, w.splits, rows, n, w.Yu, n, 1.f, 0.f, stream));
+    MPQ_HIP_TRY(splitk_reduce(w.P, w.splits, sstride, rows, n, w.Yu, n, 1.f, 0.f, stream));
   }
   // RTN error (rtn_err, and the obs warm start when none is given), from x_init Vs (or the caller's)
   if (pr.xr_in) {
