@@ -22,35 +22,54 @@ namespace {
 
 inline int64_t a64(int64_t v) { return (v + 63) / 64 * 64; }
 
-// group abs-max gmax[r][g] = max |W[r][g*gs .. (g+1)*gs)|
+// group abs-max gmax[r][g] = max |W[r][g*gs .. (g+1)*gs)|, one wave per (row, group)
 __global__ __launch_bounds__(256) void group_absmax_kernel(const float* __restrict__ W, int64_t rows, int64_t n,
                                                            int64_t gs, float* __restrict__ gmax) {
   const int64_t G = n / gs;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t idx = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (idx >= rows * G) return;
   const int64_t r = idx / G, g = idx % G;
+  const float* w = W + r * n + g * gs;
   float m = 0.f;
-  for (int64_t j = 0; j < gs; ++j) m = fmaxf(m, fabsf(W[r * n + g * gs + j]));
-  gmax[idx] = m;
+  for (int64_t j = threadIdx.x & 63; j < gs; j += 64) m = fmaxf(m, fabsf(w[j]));
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  if ((threadIdx.x & 63) == 0) gmax[idx] = m;
 }
 
-// w_sum[j] = sum_rows |W[r][j]| / (gmax[r][g(j)] + 1e-6), rows in order
-__global__ __launch_bounds__(256) void w_sum_kernel(const float* __restrict__ W, int64_t rows, int64_t n, int64_t gs,
-                                                    const float* __restrict__ gmax, float* __restrict__ w_sum) {
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
+// w_sum[j] += sum_r |W[r][j]| / (gmax + 1e-6), in a fixed order: a work-group owns 16 columns, thread (g, j) adds
+// the rows g, g + 64, ... of column j, and the 64 sums of a column are added pairwise in LDS.  (4096 x 4096: 24 us;
+// one thread per column was a chain of 4096 loads in 16 work-groups.)
+__global__ __launch_bounds__(1024) void w_sum_kernel(const float* __restrict__ W, int64_t rows, int64_t n, int64_t gs,
+                                                     const float* __restrict__ gmax, float* __restrict__ w_sum) {
+  __shared__ float red[64][17];
   const int64_t G = n / gs;
-  const int64_t g = j / gs;
+  const int c = threadIdx.x & 15, t = threadIdx.x >> 4;
+  const int64_t j = (int64_t)blockIdx.x * 16 + c;
   float acc = 0.f;
-  for (int64_t r = 0; r < rows; ++r) acc += fabsf(W[r * n + j]) / (gmax[r * G + g] + 1e-6f);
-  w_sum[j] += acc;
+  if (j < n) {
+    const int64_t g = j / gs;
+#pragma unroll 4
+    for (int64_t r = t; r < rows; r += 64) acc += fabsf(W[r * n + j]) / (gmax[r * G + g] + 1e-6f);
+  }
+  red[t][c] = acc;
+  __syncthreads();
+  for (int w = 32; w > 0; w >>= 1) {
+    if (t < w) red[t][c] += red[t + w][c];
+    __syncthreads();
+  }
+  if (t == 0 && j < n) w_sum[j] += red[0][c];
 }
 
-// candidate scales for ratio k/20 (one work-group): s = clamp(x^r / (w^(1-r) + 1e-4), 1e-4),
+constexpr int kRatios = 20;
+
+// candidate scales for the ratios k/20, one work-group each (work-group k writes s[k n ..]): s = clamp(x^r / (w^(1-r) + 1e-4), 1e-4),
 // s /= sqrt(max * min), non-finite -> 1
 __global__ __launch_bounds__(256) void candidate_scales_kernel(const float* __restrict__ x_mean,
                                                                const float* __restrict__ w_mean, int64_t n,
-                                                               float ratio, float* __restrict__ s) {
+                                                               float* __restrict__ s) {
+  const float ratio = (float)blockIdx.x / (float)kRatios;
+  s += blockIdx.x * n;
   __shared__ float smax[256], smin[256];
   float mx = -INFINITY, mn = INFINITY;
   for (int64_t j = threadIdx.x; j < n; j += blockDim.x) {
@@ -157,11 +176,37 @@ __global__ void loss_kernel(int64_t rows, const float* __restrict__ rowq, float*
 }  // namespace
 }  // namespace mpq
 
+namespace mpq {
+namespace {
+
+// The search's workspace.  The 20 products D H run as x6 products on H packed once (f16 matrix cores) where
+// the shape has them; else, and for problems so small that the launches are what counts, on the fp32 kernel.
+// 4096 x 4096, per ratio: 1.21 ms (fp32 product) -> 0.41 (x6) + 0.04 (packing D); below n = 1024 the extra
+// launches cost more than the product gains (4096 x 512, the whole search: 1.50 ms with x6, 1.20 without; 2475 x
+// 384: 1.18 / 0.94).
+struct AwqPlan {
+  bool x6;
+  int splits, bn;
+  int64_t hp_bytes, ap_bytes, bytes;
+};
+
+AwqPlan awq_plan(int64_t rows, int64_t n) {
+  AwqPlan p{};
+  p.bn = 128;
+  p.x6 = x6_shape_ok(n, n) && n >= 1024;
+  p.splits = p.x6 ? x6_choose_splits(rows, n, n) : choose_splits(rows, n, n, (int64_t)1 << 62, &p.bn);
+  p.hp_bytes = p.x6 ? a64(n * n) * 4 : 0;
+  p.ap_bytes = p.x6 ? (x6_packed_a_bytes(rows, n) + 255) / 256 * 256 : 0;
+  p.bytes = (a64(rows * n) * (1 + p.splits) + a64(rows) + 64 + a64(kRatios * n)) * 4 + p.hp_bytes + p.ap_bytes;
+  return p;
+}
+
+}  // namespace
+}  // namespace mpq
+
 extern "C" int64_t mpq_awq_workspace_size(int64_t rows, int64_t n) {
   if (rows <= 0 || n <= 0) return 0;
-  int bn = 128;
-  const int splits = mpq::choose_splits(rows, n, n, (int64_t)1 << 62, &bn);
-  return (mpq::a64(rows * n) * (1 + splits) + mpq::a64(rows) * 2 + mpq::a64(n) * 2 + 64) * 4;
+  return mpq::awq_plan(rows, n).bytes;
 }
 
 extern "C" int mpq_awq_w_mean(const float* W, int64_t rows, int64_t n, int64_t group_size, float* w_sum,
@@ -174,9 +219,9 @@ extern "C" int mpq_awq_w_mean(const float* W, int64_t rows, int64_t n, int64_t g
                 "mpq_awq_w_mean: bad pointer or workspace");
   float* gmax = static_cast<float*>(workspace);
   const int64_t cnt = rows * (n / group_size);
-  hipLaunchKernelGGL(group_absmax_kernel, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, stream, W, rows, n,
+  hipLaunchKernelGGL(group_absmax_kernel, dim3((unsigned)((cnt + 3) / 4)), dim3(256), 0, stream, W, rows, n,
                      group_size, gmax);
-  hipLaunchKernelGGL(w_sum_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, W, rows, n, group_size,
+  hipLaunchKernelGGL(w_sum_kernel, dim3((unsigned)((n + 15) / 16)), dim3(1024), 0, stream, W, rows, n, group_size,
                      gmax, w_sum);
   MPQ_LAUNCH_CHECK();
   return kOk;
@@ -193,40 +238,46 @@ extern "C" int mpq_awq_search(const float* W, int64_t rows, int64_t n, const flo
   MPQ_CHECK_ARG(W && H && x_mean && w_mean && best_scales && workspace, "mpq_awq_search: null pointer");
   MPQ_CHECK_ARG(workspace_bytes >= mpq_awq_workspace_size(rows, n), "mpq_awq_search: workspace too small");
   MPQ_CHECK_ARG(rows <= 65535 * 128LL, "mpq_awq_search: too many rows");
-  int bn = 128;
-  const int splits = choose_splits(rows, n, n, (int64_t)1 << 62, &bn);
+  const AwqPlan pl = awq_plan(rows, n);
   char* p = static_cast<char*>(workspace);
   float* D = (float*)p; p += a64(rows * n) * 4;
-  float* P = (float*)p; p += a64(rows * n) * splits * 4;
+  float* P = (float*)p; p += a64(rows * n) * pl.splits * 4;
   float* rowq = (float*)p; p += a64(rows) * 4;
-  float* losses = (float*)p; p += a64(rows) * 4;  // first 20 used
-  float* s = (float*)p; p += a64(n) * 4;
-  float* s_best = (float*)p;
+  float* losses = (float*)p; p += 64 * 4;  // first 20 used
+  float* s = (float*)p; p += a64(kRatios * n) * 4;
+  float* Hp = (float*)p; p += pl.hp_bytes;
+  void* Ap = p;
   const int64_t G = n / group_size;
   const int64_t waves = rows * G;
-  for (int k = 0; k < 20; ++k) {
-    const float ratio = (float)k / 20.0f;
-    hipLaunchKernelGGL(candidate_scales_kernel, dim3(1), dim3(256), 0, stream, x_mean, w_mean, n, ratio, s);
+  hipLaunchKernelGGL(candidate_scales_kernel, dim3(kRatios), dim3(256), 0, stream, x_mean, w_mean, n, s);
+  MPQ_LAUNCH_CHECK();
+  if (pl.x6) MPQ_HIP_TRY(x6_pack_b(H, n, false, n, n, Hp, stream));
+  for (int k = 0; k < kRatios; ++k) {
     hipLaunchKernelGGL(awq_delta_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, W, rows, n,
-                       group_size, s, bits, sym ? 1 : 0, D);
+                       group_size, s + k * n, bits, sym ? 1 : 0, D);
     MPQ_LAUNCH_CHECK();
-    GemmParams gp{};
-    gp.M = rows; gp.N = n; gp.K = n;
-    gp.A = D; gp.lda = n; gp.B = H; gp.ldb = n; gp.trans_b = false;
-    gp.C = P; gp.ldc = n; gp.split_stride = a64(rows * n);
-    gp.alpha = 1.f; gp.beta = 0.f; gp.mode = kGemmPartials;
-    MPQ_HIP_TRY(gemm_partials(gp, splits, bn, stream));
-    hipLaunchKernelGGL(row_quad_kernel, dim3((unsigned)rows), dim3(256), 0, stream, n, P, splits, a64(rows * n), D,
+    if (pl.x6) {
+      MPQ_HIP_TRY(x6_pack_a(D, n, rows, n, Ap, stream));
+      MPQ_HIP_TRY(x6_gemm_partials(Ap, Hp, rows, n, n, P, n, a64(rows * n), pl.splits, stream));
+    } else {
+      GemmParams gp{};
+      gp.M = rows; gp.N = n; gp.K = n;
+      gp.A = D; gp.lda = n; gp.B = H; gp.ldb = n; gp.trans_b = false;
+      gp.C = P; gp.ldc = n; gp.split_stride = a64(rows * n);
+      gp.alpha = 1.f; gp.beta = 0.f; gp.mode = kGemmPartials;
+      MPQ_HIP_TRY(gemm_partials(gp, pl.splits, pl.bn, stream));
+    }
+    hipLaunchKernelGGL(row_quad_kernel, dim3((unsigned)rows), dim3(256), 0, stream, n, P, pl.splits, a64(rows * n), D,
                        rowq);
     hipLaunchKernelGGL(loss_kernel, dim3(1), dim3(256), 0, stream, rows, rowq, losses + k);
     MPQ_LAUNCH_CHECK();
   }
-  float hl[20];
+  float hl[kRatios];
   MPQ_HIP_TRY(hipMemcpyAsync(hl, losses, sizeof(hl), hipMemcpyDeviceToHost, stream));
   MPQ_HIP_TRY(hipStreamSynchronize(stream));
   int best = -1;
   float be = INFINITY;
-  for (int k = 0; k < 20; ++k) {
+  for (int k = 0; k < kRatios; ++k) {
     if (hl[k] < be) {
       be = hl[k];
       best = k;
@@ -237,13 +288,10 @@ extern "C" int mpq_awq_search(const float* W, int64_t rows, int64_t n, const flo
     set_error_code(kNumerical);
     return kNumerical;
   }
-  hipLaunchKernelGGL(candidate_scales_kernel, dim3(1), dim3(256), 0, stream, x_mean, w_mean, n,
-                     (float)best / 20.0f, s_best);
-  MPQ_LAUNCH_CHECK();
-  MPQ_HIP_TRY(hipMemcpyAsync(best_scales, s_best, n * 4, hipMemcpyDeviceToDevice, stream));
+  MPQ_HIP_TRY(hipMemcpyAsync(best_scales, s + best * n, n * 4, hipMemcpyDeviceToDevice, stream));
   if (losses_out) MPQ_HIP_TRY(hipMemcpyAsync(losses_out, hl, sizeof(hl), hipMemcpyHostToDevice, stream));
   MPQ_HIP_TRY(hipStreamSynchronize(stream));
   if (best_error) *best_error = be;
-  if (best_ratio) *best_ratio = (float)best / 20.0f;
+  if (best_ratio) *best_ratio = (float)best / (float)kRatios;
   return kOk;
 }
