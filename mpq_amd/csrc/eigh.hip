@@ -333,7 +333,12 @@ __device__ __forceinline__ void block_sum3(T& a, T& b, T& c, T (*scratch)[kThr /
 // g = r + 32 blockIdx + tid / 8: lane k adds the symv partials of strips b0 + k, b0 + k + 8, ...,
 // chunks k, k + 8, ... and the reflectors j = k, k + 8, ...; a fixed butterfly over the eight
 // lanes completes the sums.
-template <typename T>
+//
+// kPv, kPr: batched loads per thread of the x^T A x and the symv partials.  A fixed large batch (32 and 32, for
+// trailing matrices up to 16384 rows) costs a small one its issue time: a
+// solve took 41.0 ms at n = 2048 in fp64 with them and takes 34.2, 14.5 / 12.2 at n = 903 in fp32, 336 / 313 at
+// n = 8192 in fp64.
+template <typename T, int kPv, int kPr>
 __global__ __launch_bounds__(kThr) void finish_kernel(T* __restrict__ A, int64_t lda, int64_t n, int64_t c,
                                                      int64_t i0, int i, int do_next, T* __restrict__ alph,
                                                      const T* __restrict__ Pn_in, int npn,
@@ -357,9 +362,8 @@ __global__ __launch_bounds__(kThr) void finish_kernel(T* __restrict__ A, int64_t
   // Every global load of the kernel is issued in one batch before any of them is used: fixed-size,
   // unrolled batches from clamped in-range addresses whose values are selected afterwards.  (A
   // guarded load, or a loop that accumulates while it loads, costs a memory round trip each.)
-  // Only trailing matrices above 2 kThr norm partials, kPvBatch kThr symv partials or 32 kSub
+  // Only trailing matrices above 2 kThr norm partials, kPv kThr x^T A x partials or kPr kSub
   // strips take the remainder loops below.
-  constexpr int kPvBatch = 32;
   const int npv = chy * ns;  // x^T A x partials (chunk, strip); some slots hold no chunk
   const int gl = (int)min(g, n - 1);  // in-range row for the loads of inactive threads
   const int s_row = gl / kTB;
@@ -375,13 +379,13 @@ __global__ __launch_bounds__(kThr) void finish_kernel(T* __restrict__ A, int64_t
   // partial idx = tid + kThr u sits at (chunk idx / ns, strip b0 + idx % ns); both indices step
   // by a fixed quotient and remainder (no division per element).  pv_ok bit u: the slot holds a
   // chunk (strip sx has a chunk chx when sx < ns - chl chx).
-  T pv_v[kPvBatch];
+  T pv_v[kPv];
   unsigned pv_ok = 0u;
   {
     const int q_step = kThr / ns, r_step = kThr % ns;
     int chx = tid / ns, sx = tid % ns;
 #pragma unroll
-    for (int u = 0; u < kPvBatch; ++u) {
+    for (int u = 0; u < kPv; ++u) {
       const int idx = tid + kThr * u;
       pv_v[u] = 0.f;
       if (idx < npv) {
@@ -402,9 +406,9 @@ __global__ __launch_bounds__(kThr) void finish_kernel(T* __restrict__ A, int64_t
   const T svr_v = A[(i0 + jr) * lda + r];
   const T swr_v = Wb[(int64_t)jr * lda + r];
   const T arr = A[r * lda + r];
-  T pr_v[32];
+  T pr_v[kPr];
 #pragma unroll
-  for (int q = 0; q < 32; ++q) pr_v[q] = Pr[(int64_t)min(b0 + k + kSub * q, s_row) * lda + gl];
+  for (int q = 0; q < kPr; ++q) pr_v[q] = Pr[(int64_t)min(b0 + k + kSub * q, s_row) * lda + gl];
   T pc_v[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q)
@@ -428,9 +432,9 @@ __global__ __launch_bounds__(kThr) void finish_kernel(T* __restrict__ A, int64_t
   for (int u = 0; u < kDotWG / 4; ++u) pqp += pq_v[u];
   T xux = 0.f;
 #pragma unroll
-  for (int u = 0; u < kPvBatch; ++u)
+  for (int u = 0; u < kPv; ++u)
     if (pv_ok & (1u << u)) xux += pv_v[u];
-  for (int idx = tid + kThr * kPvBatch; idx < npv; idx += kThr) {
+  for (int idx = tid + kThr * kPv; idx < npv; idx += kThr) {
     const int chx = idx / ns, sx = idx % ns;
     if (sx < ns - chl * chx) xux += Pvv[(int64_t)chx * nblk + b0 + sx];
   }
@@ -446,9 +450,9 @@ __global__ __launch_bounds__(kThr) void finish_kernel(T* __restrict__ A, int64_t
   T u = 0.f;
   if (active) {
 #pragma unroll
-    for (int q = 0; q < 32; ++q)
+    for (int q = 0; q < kPr; ++q)
       if (b0 + k + kSub * q <= s_row) u += pr_v[q];
-    for (int bj = b0 + k + 32 * kSub; bj <= s_row; bj += kSub) u += Pr[(int64_t)bj * lda + g];
+    for (int bj = b0 + k + kPr * kSub; bj <= s_row; bj += kSub) u += Pr[(int64_t)bj * lda + g];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
       if (k + kSub * q < nch) u += pc_v[q];
@@ -762,7 +766,11 @@ int sytrd(int64_t n, const SyevdLayout& L, T* base, hipStream_t stream) {
       MPQ_LAUNCH_CHECK();
       const int do_next = (i + 1 < nbl) || (c + 1 == n - 1);
       const int fblocks = (int)((n - c - 1 + kRowsPB - 1) / kRowsPB);
-      hipLaunchKernelGGL(finish_kernel<T>, dim3((unsigned)fblocks), dim3(kThr), 0, stream, A, lda, n, c, i0, i,
+      // batches that hold the strips (kSub per load) and the partials chy ns (kThr per load)
+      const auto finish = ns <= 16 ? finish_kernel<T, 1, 2> : ns <= 32 ? finish_kernel<T, 4, 4>
+                        : ns <= 64 ? finish_kernel<T, 4, 8> : ns <= 128 ? finish_kernel<T, 16, 16>
+                                                                        : finish_kernel<T, 32, 32>;
+      hipLaunchKernelGGL(finish, dim3((unsigned)fblocks), dim3(kThr), 0, stream, A, lda, n, c, i0, i,
                          do_next, alph, pn_in, npn, pn_out, Wb, Pr, Pc, Pvv, Ppq, ch_alloc, chl, D, E, tau);
       MPQ_LAUNCH_CHECK();
       npn = fblocks;

@@ -184,3 +184,18 @@ def test_eigen_cache_exact_match_only(gpu):
     assert e[2] is not d[2]
     assert torch.equal(e[2], d[2]) and torch.equal(e[0], d[0])  # deterministic: same bits either way
     clear_eigen_cache()
+
+
+@pytest.mark.parametrize("n,dtype", [(1025, torch.float32), (1090, torch.float64), (2048, torch.float64),
+                                     (2115, torch.float64)])
+def test_one_stage_batch_sizes(gpu, n, dtype):
+    """The finishing kernel's load batches change at 16, 32, 64 and 128 strips of 64 rows left: solves that
+    cross them, against the matrix itself (backward error and orthogonality n u, u the unit roundoff)."""
+    g = torch.Generator().manual_seed(n)
+    A = torch.randn(n, n, generator=g, dtype=torch.float64)
+    H = ((A + A.T) / 2).to(dtype).to(gpu)
+    lam, V = ops.syevd(H, method=1)
+    u = 2.0 ** -24 if dtype == torch.float32 else 2.0 ** -53
+    Hd, Vd = H.double(), V.double()
+    assert float((Hd @ Vd - Vd * lam.double()).norm()) <= n * u * float(Hd.norm())
+    assert float((Vd.T @ Vd - torch.eye(n, device=gpu, dtype=torch.float64)).norm()) <= n * u * n ** 0.5
