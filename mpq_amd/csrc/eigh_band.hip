@@ -1504,7 +1504,8 @@ __global__ __launch_bounds__(kThr) void q2_build_kernel(const float* __restrict_
 // Bound at n = 14336: memory and L2 traffic (two thirds of the time goes with the rows of Zq, a fifth with P
 // where it misses the L2; the products need 19 ms).  With six bf16 products, three planes, four groups in flight and
 // Zq as one matrix (rows 57344 bytes apart) a solve took 409 ms, with f16 pairs 393, with eight groups and strips
-// 386; n = 4096 63.3 / 62.1 / 61.3.
+// 386; n = 4096 63.3 / 62.1 / 61.3.  On another card 398 against 395 at n = 14336 (this kernel 89 and 88 ms of
+// it) and 65.3 against 63.5 at 4096.
 constexpr int kQ2Waves = 8;  // groups in flight per work-group
 constexpr int kQ2Pad = 128;  // zero rows below the matrix (prefetches past a group's end read them)
 constexpr int kQ2Cols = 64;   // columns of a strip
