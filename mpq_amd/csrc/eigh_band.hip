@@ -37,7 +37,6 @@
 // bulges need), with zero columns past n - 1 so the last tasks read and write zeros there.
 #include "eigh_band.h"
 #include "gemm.h"
-#include "f16_pair.h"
 #include "x6_split.h"
 
 namespace mpq {
@@ -46,7 +45,6 @@ namespace {
 
 constexpr int kThr = 256;
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ void wave_sync() {
@@ -1421,17 +1419,13 @@ __global__ __launch_bounds__(kThr) void tridiag_out_kernel(const float* __restri
 
 // ---- back-transformation of stage 2 ----------------------------------------------------------
 
-constexpr int kPtChunks = 2 * 512;  // uint4 per block: 2 f16 planes x (2 row tiles x 4 k-steps x 64 lanes)
-// P and the eigenvectors are orthogonal, so their entries are at most 1 in magnitude (to rounding): a
-// fixed scale of 2^14 keeps both planes of a pair (f16_pair.h) in f16's normal range down to 2^-16, and below that
-// the representation error is 2^-39 at most.  Results carry 2^28.
-constexpr float kQ2Scale = 0x1p14f, kQ2Unscale = 0x1p-28f, kQ2Rescale = 0x1p-14f;
+constexpr int kPtChunks = 3 * 512;  // uint4 per block: 3 bf16 planes x (2 row tiles x 4 k-steps x 64 lanes)
 
 // Block (g, k): P = (H_31 ... H_0)^T over the window rows 32 g + 1 + 32 k .. + 63, H_i the reflector
 // of sweep 32 g + i at step k (acting on window rows i .. i + 31; identity where it does not
 // exist).  One work-group per block; thread (c = t % 64, q = t / 64) owns column c, rows q (mod 4)
-// of M = H_31 ... H_0, then P = M^T leaves as a pair of scaled f16 planes (to 2^-23) in the
-// left-operand order of v_mfma_f32_32x32x16_f16 with the k index permuted: chunk (plane, tile,
+// of M = H_31 ... H_0, then P = M^T leaves as three bf16 planes (P = P0 + P1 + P2 to 2^-24) in the
+// left-operand order of v_mfma_f32_32x32x16_bf16 with the k index permuted: chunk (plane, tile,
 // step, lane) holds the 8 entries P[32 tile + lane % 32][16 step + 8 (j / 4) + 4 (lane / 32) + j % 4],
 // j = 0 .. 7 (the window row that k slot j of the lane stands for in q2_apply_kernel).
 __global__ __launch_bounds__(kThr) void q2_build_kernel(const float* __restrict__ V2, const float* __restrict__ tau2,
@@ -1475,45 +1469,40 @@ __global__ __launch_bounds__(kThr) void q2_build_kernel(const float* __restrict_
   for (int ci = t; ci < 512; ci += kThr) {
     const int l = ci & 63, ts = ci >> 6;
     const int cc = 32 * (ts >> 2) + (l & 31), k0 = 16 * (ts & 3) + 4 * (l >> 5);
-    uint32_t h[4], lo[4];
+    uint32_t h[4], m[4], lo[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int kk = k0 + 2 * (j & 1) + 8 * (j >> 1);  // slots 2 j, 2 j + 1
-      split2(M[kk][cc], M[kk + 1][cc], kQ2Scale, h[j], lo[j]);
+      split3(M[kk][cc], M[kk + 1][cc], h[j], m[j], lo[j]);
     }
     out[ci] = make_uint4(h[0], h[1], h[2], h[3]);
-    out[512 + ci] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    out[512 + ci] = make_uint4(m[0], m[1], m[2], m[3]);
+    out[1024 + ci] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
   }
 }
 
 
-// Zq (strips of 64 columns, each (n + kQ2Pad) x 64 row-major, zero outside the n x n matrix; column j =
-// eigenvector j of the tridiagonal matrix) <- Q2 Zq: groups last to first, blocks in increasing order, each block
+// Zq ((n + kQ2Pad) x ldq, row-major, zero outside the n x n matrix; column j = eigenvector j of
+// the tridiagonal matrix) <- Q2 Zq: groups last to first, blocks in increasing order, each block
 // Zq[lo .. lo + 63][:] <- P(g, k) Zq[lo .. lo + 63][:].  One work-group per 64 columns and one wave
-// per group: eight groups at once (two waves per SIMD), group gl - q on wave q.  Block k of group g reads rows that
+// per group: four groups at once, group gl - q on wave q.  Block k of group g reads rows that
 // block k - 1 of group g + 1 (wave q - 1) finishes, and its prefetch two blocks ahead the rows of
 // block k + 1 of group g + 1: each wave publishes its last finished block in LDS and waits for
 // its predecessor's before loading rows.  A wave keeps the whole 64 x 64 block result in
-// registers (four 32 x 32 tiles; K = 64 as four 16-k steps; three f16 plane products each): the
-// finished upper half goes to memory, while the lower half, split into f16 pairs in registers,
+// registers (four 32 x 32 tiles; K = 64 as four 16-k steps; six bf16 plane products each): the
+// finished upper half goes to memory, while the lower half, split into bf16 planes in registers,
 // is the next block's upper window as it stands, because P's columns are packed in the order that
 // lines each result register up with the right-operand slot holding the same row: k slot (s, h, j)
 // of lane l (h = l / 32) is window row 16 s + 8 (j / 4) + 4 h + j % 4.  The window's new rows load
 // from memory straight into that order.  No data passes through LDS and waves do not wait on one
 // another except for rows.
-// Bound at n = 14336: memory and L2 traffic (two thirds of the time goes with the rows of Zq, a fifth with P
-// where it misses the L2; the products need 19 ms).  With six bf16 products, three planes, four groups in flight and
-// Zq as one matrix (rows 57344 bytes apart) a solve took 409 ms, with f16 pairs 393, with eight groups and strips
-// 386; n = 4096 63.3 / 62.1 / 61.3.  On another card 398 against 395 at n = 14336 (this kernel 89 and 88 ms of
-// it) and 65.3 against 63.5 at 4096.
-constexpr int kQ2Waves = 8;  // groups in flight per work-group
 constexpr int kQ2Pad = 128;  // zero rows below the matrix (prefetches past a group's end read them)
-constexpr int kQ2Cols = 64;   // columns of a strip
+static_assert((kMaxN + kQ2Pad) * ((kMaxN + 63) / 64 * 64) * 4 < ((int64_t)1 << 31), "Zq byte offsets are int32");
 
 struct Q2Ops {
-  uint4 a01[1][2][2][2];  // P planes, k steps 0, 1 [-][row tile][k step][plane]
-  uint4 a23[2][2][2];     // P planes, k steps 2, 3 [row tile][k step - 2][plane]
-  uint4 b[2][4][2];    // window planes [column tile][k step][plane]
+  uint4 a01[1][2][2][3];  // P planes, k steps 0, 1 [-][row tile][k step][plane]
+  uint4 a23[2][2][3];     // P planes, k steps 2, 3 [row tile][k step - 2][plane]
+  uint4 b[2][4][3];    // window planes [column tile][k step][plane]
   floatx16 acc[2][2];  // block result [row tile][column tile]
   float raw[2][2][8];  // window rows (32 + 16 s' .. of a later block) [column tile][s'][slot]
 };
@@ -1523,7 +1512,7 @@ struct Q2Ops {
 struct Q2Wave {
   const uint4* Pt;
   __amdgpu_buffer_rsrc_t rz;  // Zq
-  int vz[2];                  // lane byte offset, column tile ct: row 4 (lane / 32), column 32 ct + lane % 32
+  int vz[2];                  // lane byte offset, column tile ct: row 4 (lane / 32), column z0 + 32 ct + lane % 32
   int ldq4;                   // bytes per row of Zq
   int roff[16];               // byte offset of row 8 (i / 4) + i % 4 (k slots 8 s + j, result registers v)
   int lane;
@@ -1544,7 +1533,7 @@ __device__ __forceinline__ void q2w_load_a(Q2Ops& o, const Q2Wave& w, int64_t bi
 #pragma unroll
     for (int s = S0; s < S0 + 2; ++s)
 #pragma unroll
-      for (int p = 0; p < 2; ++p) {
+      for (int p = 0; p < 3; ++p) {
         const uint4 v = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                                       r, vo, (p * 512 + (rt * 4 + s) * 64) * 16, 0));
         if (S0 == 0) o.a01[SET][rt][s][p] = v;
@@ -1563,11 +1552,11 @@ __device__ __forceinline__ void q2w_load_rows(Q2Ops& o, const Q2Wave& w, int row
   }
 }
 
-__device__ __forceinline__ void q2w_split8(const float* x, float scale, uint4 (&pl)[2]) {
-  split2(x[0], x[1], scale, pl[0].x, pl[1].x);
-  split2(x[2], x[3], scale, pl[0].y, pl[1].y);
-  split2(x[4], x[5], scale, pl[0].z, pl[1].z);
-  split2(x[6], x[7], scale, pl[0].w, pl[1].w);
+__device__ __forceinline__ void q2w_split8(const float* x, uint4& h, uint4& m, uint4& l) {
+  split3(x[0], x[1], h.x, m.x, l.x);
+  split3(x[2], x[3], h.y, m.y, l.y);
+  split3(x[4], x[5], h.z, m.z, l.z);
+  split3(x[6], x[7], h.w, m.w, l.w);
 }
 
 // k steps SB, SB + 1 of the window from the loaded rows
@@ -1576,7 +1565,7 @@ __device__ __forceinline__ void q2w_split_rows(Q2Ops& o) {
 #pragma unroll
   for (int ct = 0; ct < 2; ++ct)
 #pragma unroll
-    for (int s = 0; s < 2; ++s) q2w_split8(o.raw[ct][s], kQ2Scale, o.b[ct][SB + s]);
+    for (int s = 0; s < 2; ++s) q2w_split8(o.raw[ct][s], o.b[ct][SB + s][0], o.b[ct][SB + s][1], o.b[ct][SB + s][2]);
 }
 
 // k steps 0, 1 of the next window from the lower result tile: result register 8 s + j of the lane
@@ -1589,20 +1578,23 @@ __device__ __forceinline__ void q2w_split_lower(Q2Ops& o) {
       float x[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = o.acc[1][ct][8 * s + j];
-      q2w_split8(x, kQ2Rescale, o.b[ct][s]);  // a result carries the scale twice
+      q2w_split8(x, o.b[ct][s][0], o.b[ct][s][1], o.b[ct][s][2]);
     }
 }
 
-// row tile RT, k step S: three plane products into both column tiles (FRESH: the first k step)
+// row tile RT, k step S: six plane products into both column tiles (FRESH: the first k step)
 template <int SET, int RT, int S, bool FRESH>
 __device__ __forceinline__ void q2w_mfma(Q2Ops& o) {
   const uint4* pa = S < 2 ? o.a01[SET][RT][S] : o.a23[RT][S - 2];
-  const f16x8 a0 = __builtin_bit_cast(f16x8, pa[0]);
-  const f16x8 a1 = __builtin_bit_cast(f16x8, pa[1]);
-  const f16x8 b0 = __builtin_bit_cast(f16x8, o.b[0][S][0]);
-  const f16x8 b1 = __builtin_bit_cast(f16x8, o.b[0][S][1]);
-  const f16x8 d0 = __builtin_bit_cast(f16x8, o.b[1][S][0]);
-  const f16x8 d1 = __builtin_bit_cast(f16x8, o.b[1][S][1]);
+  const bf16x8 a0 = __builtin_bit_cast(bf16x8, pa[0]);
+  const bf16x8 a1 = __builtin_bit_cast(bf16x8, pa[1]);
+  const bf16x8 a2 = __builtin_bit_cast(bf16x8, pa[2]);
+  const bf16x8 b0 = __builtin_bit_cast(bf16x8, o.b[0][S][0]);
+  const bf16x8 b1 = __builtin_bit_cast(bf16x8, o.b[0][S][1]);
+  const bf16x8 b2 = __builtin_bit_cast(bf16x8, o.b[0][S][2]);
+  const bf16x8 d0 = __builtin_bit_cast(bf16x8, o.b[1][S][0]);
+  const bf16x8 d1 = __builtin_bit_cast(bf16x8, o.b[1][S][1]);
+  const bf16x8 d2 = __builtin_bit_cast(bf16x8, o.b[1][S][2]);
   floatx16 c0, c1;
   if (FRESH) {
 #pragma unroll
@@ -1614,12 +1606,18 @@ __device__ __forceinline__ void q2w_mfma(Q2Ops& o) {
     c0 = o.acc[RT][0];
     c1 = o.acc[RT][1];
   }
-  c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b0, c0, 0, 0, 0);
-  c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, d0, c1, 0, 0, 0);
-  c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b1, c0, 0, 0, 0);
-  c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, d1, c1, 0, 0, 0);
-  c0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b0, c0, 0, 0, 0);
-  c1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, d0, c1, 0, 0, 0);
+  c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b0, c0, 0, 0, 0);
+  c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, d0, c1, 0, 0, 0);
+  c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b1, c0, 0, 0, 0);
+  c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, d1, c1, 0, 0, 0);
+  c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b0, c0, 0, 0, 0);
+  c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, d0, c1, 0, 0, 0);
+  c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, b2, c0, 0, 0, 0);
+  c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0, d2, c1, 0, 0, 0);
+  c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, c0, 0, 0, 0);
+  c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, d1, c1, 0, 0, 0);
+  c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a2, b0, c0, 0, 0, 0);
+  c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a2, d0, c1, 0, 0, 0);
   o.acc[RT][0] = c0;
   o.acc[RT][1] = c1;
 }
@@ -1630,8 +1628,8 @@ __device__ __forceinline__ void q2w_store(const floatx16 (&c)[2], const Q2Wave& 
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
     const int so = rb + w.roff[v];
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(c[0][v] * kQ2Unscale), w.rz, w.vz[0], so, 0);
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(c[1][v] * kQ2Unscale), w.rz, w.vz[1], so, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(c[0][v]), w.rz, w.vz[0], so, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(c[1][v]), w.rz, w.vz[1], so, 0);
   }
 }
 
@@ -1679,7 +1677,7 @@ __device__ __forceinline__ void q2w_block(Q2Ops& o, Q2Wave& w, int k, int nk, in
     q2w_split_lower(o);
     q2w_mfma<SET, 0, 3, false>(o);
 #pragma unroll
-    for (int i = 0; i < 12; ++i) {
+    for (int i = 0; i < 24; ++i) {
       __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 0);
       __builtin_amdgcn_sched_group_barrier(kSgValu, 10, 0);
     }
@@ -1692,8 +1690,8 @@ __device__ __forceinline__ void q2w_block(Q2Ops& o, Q2Wave& w, int k, int nk, in
   q2w_mfma<SET, 1, 3, false>(o);
   q2w_load_a<SET, 2>(o, w, base + min(k + 1, nk - 1));
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 0);
+  for (int i = 0; i < 12; ++i) {
+    __builtin_amdgcn_sched_group_barrier(kSgMfma, 2, 0);
     __builtin_amdgcn_sched_group_barrier(kSgVmemRd, 1, 0);
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -1701,9 +1699,9 @@ __device__ __forceinline__ void q2w_block(Q2Ops& o, Q2Wave& w, int k, int nk, in
   q2w_mfma<SET, 1, 0, false>(o);
   q2w_split_rows<2>(o);  // block k + 1's k steps 2, 3
 #pragma unroll
-  for (int i = 0; i < 12; ++i) {
+  for (int i = 0; i < 24; ++i) {
     __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(kSgValu, 10, 0);
+    __builtin_amdgcn_sched_group_barrier(kSgValu, 8, 0);
   }
   __builtin_amdgcn_sched_barrier(0);
   // rows of block k + 2's k steps 2, 3 (block k + 1 of wave q - 1; clamped past the group's end)
@@ -1713,24 +1711,25 @@ __device__ __forceinline__ void q2w_block(Q2Ops& o, Q2Wave& w, int k, int nk, in
   q2w_mfma<SET, 1, 1, false>(o);
   q2w_load_a<0, 0>(o, w, base + min(k + 1, nk - 1));
 #pragma unroll
-  for (int i = 0; i < 12; ++i) {
+  for (int i = 0; i < 22; ++i) {
     __builtin_amdgcn_sched_group_barrier(kSgMfma, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(kSgVmemRd, 4, 0);
+    __builtin_amdgcn_sched_group_barrier(kSgVmemRd, 2, 0);
   }
 }
 
-__global__ __launch_bounds__(64 * kQ2Waves, 2) void q2_apply_kernel(const uint4* __restrict__ Pt, float* __restrict__ Zq,
-                                                       int64_t n64, int* __restrict__ status) {
-  __shared__ int sprog[kQ2Waves];
+__global__ __launch_bounds__(256) void q2_apply_kernel(const uint4* __restrict__ Pt, float* __restrict__ Zq,
+                                                       int64_t n64, int64_t ldq, int* __restrict__ status) {
+  __shared__ int sprog[4];
   const int t = threadIdx.x, lane = t & 63;
   const int q = __builtin_amdgcn_readfirstlane(t >> 6);
   const int n = (int)n64;
+  const int z0 = (int)blockIdx.x * 64;
   Q2Wave w;
   w.Pt = Pt;
-  const int64_t strip = (n64 + kQ2Pad) * kQ2Cols;
-  w.rz = __builtin_amdgcn_make_buffer_rsrc(Zq + blockIdx.x * strip, (short)0, (int)(strip * 4), 0x00020000);
-  w.ldq4 = kQ2Cols * 4;
-  w.vz[0] = (4 * (lane >> 5) * kQ2Cols + (lane & 31)) * 4;
+  // every byte offset fits in 32 bits: (n + kQ2Pad) ldq 4 < 2^31 for n <= kMaxN
+  w.rz = __builtin_amdgcn_make_buffer_rsrc(Zq, (short)0, (int)((n64 + kQ2Pad) * ldq * 4), 0x00020000);
+  w.ldq4 = (int)ldq * 4;
+  w.vz[0] = (4 * (lane >> 5) * (int)ldq + z0 + (lane & 31)) * 4;
   w.vz[1] = w.vz[0] + 32 * 4;
 #pragma unroll
   for (int i = 0; i < 16; ++i) w.roff[i] = (8 * (i >> 2) + (i & 3)) * w.ldq4;
@@ -1741,8 +1740,8 @@ __global__ __launch_bounds__(64 * kQ2Waves, 2) void q2_apply_kernel(const uint4*
   w.failed = false;
   const int K0 = (n - 2) / kBW;
   Q2Ops o;
-  for (int gl = K0; gl >= 0; gl -= kQ2Waves) {
-    if (t < kQ2Waves) sprog[t] = -1;
+  for (int gl = K0; gl >= 0; gl -= 4) {
+    if (t < 4) sprog[t] = -1;
     __syncthreads();
     const int g = gl - q;
     if (g >= 0) {
@@ -1774,7 +1773,7 @@ __global__ __launch_bounds__(64 * kQ2Waves, 2) void q2_apply_kernel(const uint4*
 
 // Z (n x n, row j = eigenvector j) -> Zq (row i = coordinate i, zero outside n x n) and back
 __global__ __launch_bounds__(256) void q2_gather_kernel(const float* __restrict__ Z, int64_t n, float* __restrict__ Zq,
-                                                        int64_t strip) {
+                                                        int64_t ldq) {
   __shared__ float tile[32][33];
   const int64_t r0 = (int64_t)blockIdx.y * 32, c0 = (int64_t)blockIdx.x * 32;  // Zq tile
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
@@ -1783,18 +1782,17 @@ __global__ __launch_bounds__(256) void q2_gather_kernel(const float* __restrict_
     tile[i][tx] = (j < n && r < n) ? Z[j * n + r] : 0.f;
   }
   __syncthreads();
-  float* out = Zq + c0 / kQ2Cols * strip + c0 % kQ2Cols;
-  for (int i = ty; i < 32; i += 8) out[(r0 + i) * kQ2Cols + tx] = tile[tx][i];
+  for (int i = ty; i < 32; i += 8) Zq[(r0 + i) * ldq + c0 + tx] = tile[tx][i];
 }
 
-__global__ __launch_bounds__(256) void q2_scatter_kernel(const float* __restrict__ Zq, int64_t strip, int64_t n,
+__global__ __launch_bounds__(256) void q2_scatter_kernel(const float* __restrict__ Zq, int64_t ldq, int64_t n,
                                                          float* __restrict__ Z) {
   __shared__ float tile[32][33];
   const int64_t j0 = (int64_t)blockIdx.y * 32, r0 = (int64_t)blockIdx.x * 32;  // Z tile
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   for (int i = ty; i < 32; i += 8) {
     const int64_t r = r0 + i, j = j0 + tx;  // Zq[r][j]
-    tile[i][tx] = (r < n && j < n) ? Zq[j / kQ2Cols * strip + r * kQ2Cols + j % kQ2Cols] : 0.f;
+    tile[i][tx] = (r < n && j < n) ? Zq[r * ldq + j] : 0.f;
   }
   __syncthreads();
   for (int i = ty; i < 32; i += 8) {
@@ -2006,19 +2004,18 @@ int q2_apply(int64_t n, float* Z, float* ws, const Layout& L, hipStream_t stream
   const int64_t nb = q2_blocks(n);
   uint4* Pt = reinterpret_cast<uint4*>(ws + L.Pt);
   float* Zq = ws + L.Zq;
-  const int64_t strip = (n + kQ2Pad) * kQ2Cols;
   hipLaunchKernelGGL(q2_build_kernel, dim3((unsigned)nb), dim3(kThr), 0, stream, ws + L.V2, ws + L.tau2, n, Pt);
   MPQ_LAUNCH_CHECK();
   hipLaunchKernelGGL(q2_gather_kernel, dim3((unsigned)(L.ldq / 32), (unsigned)((n + kQ2Pad) / 32)), dim3(kThr), 0,
-                     stream, Z, n, Zq, strip);
+                     stream, Z, n, Zq, L.ldq);
   MPQ_LAUNCH_CHECK();
   int* status = reinterpret_cast<int*>(ws + L.prog) + (n - 1 + kNW - 1) / kNW + 1;
   hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(kThr), 0, stream, status, 1, 0);
   MPQ_LAUNCH_CHECK();
-  hipLaunchKernelGGL(q2_apply_kernel, dim3((unsigned)(L.ldq / 64)), dim3(64 * kQ2Waves), 0, stream, Pt, Zq, n, status);
+  hipLaunchKernelGGL(q2_apply_kernel, dim3((unsigned)(L.ldq / 64)), dim3(kThr), 0, stream, Pt, Zq, n, L.ldq, status);
   MPQ_LAUNCH_CHECK();
   hipLaunchKernelGGL(q2_scatter_kernel, dim3((unsigned)((n + 31) / 32), (unsigned)((n + 31) / 32)), dim3(kThr), 0,
-                     stream, Zq, strip, n, Z);
+                     stream, Zq, L.ldq, n, Z);
   MPQ_LAUNCH_CHECK();
   int st = 0;
   MPQ_HIP_TRY(hipMemcpyAsync(&st, status, sizeof(int), hipMemcpyDeviceToHost, stream));
