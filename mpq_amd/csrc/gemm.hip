@@ -754,15 +754,9 @@ int choose_splits(int64_t M, int64_t N, int64_t K, int64_t workspace_floats, int
   const int64_t tiles = tiles_m * ((N + bn - 1) / bn);
   int splits = 1;
   const int64_t target = 2048;  // ~8 work-groups per CU on 256 CUs (latency hiding at small M)
-  // Slices of at least 256, or down to 32 as long as the grid has no more than one work-group per CU: a small
-  // product is a chain of K slabs in too few work-groups.  One VAMP row block, us with the slices of 256 and
-  // with these: 104 x 1000 x 1000 35.0 / 9.2, 128 x 1024 x 1024 12.5 / 6.8, 128 x 512 x 512 12.0 / 4.7,
-  // 128 x 256 x 256 12.1 / 4.2; 128 x 2048 x 2048 takes 8 splits either way (14.2; 15.3 with 16).
-  auto more = [&](int s) {
-    const int64_t wgs = tiles * s, slice = K / s;
-    return (wgs <= target && slice >= 256) || (wgs <= 256 && slice >= 32);
-  };
-  while (splits < 32 && more(splits * 2) && (int64_t)(splits * 2) * M * N <= workspace_floats) splits *= 2;
+  while (splits < 32 && tiles * splits * 2 <= target && K / (splits * 2) >= 256 &&
+         (int64_t)(splits * 2) * M * N <= workspace_floats)
+    splits *= 2;
   *bn_out = bn;
   return splits;
 }

@@ -50,7 +50,7 @@ def stops(n, seed, device):
 
 
 # two-stage decomposition, fp32 products
-@pytest.mark.parametrize("n,seed", [(2048, 73), (2048, 79)])
+@pytest.mark.parametrize("n,seed", [(2048, 73), (2048, 79), (1536, 10), (2048, 43), (2048, 75)])
 def test_row_blocks_stop_where_they_did(gpu, n, seed):
     with open(GOLDEN) as f:
         want = json.load(f)[f"{n} {seed}"]

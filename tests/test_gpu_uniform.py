@@ -380,16 +380,3 @@ def test_vamp_early_stop_then_call_on_another_stream(gpu):
         assert torch.equal(got[0], ref[0])
         assert torch.equal(got[2], ref[2])
         assert got[4]["stop_iter"] == ref[4]["stop_iter"] and got[4]["best_iter"] == ref[4]["best_iter"]
-
-
-@pytest.mark.parametrize("M,N,K", [(104, 1000, 1000), (128, 256, 256), (1, 64, 64), (24, 104, 104), (129, 72, 2081),
-                                   (128, 512, 544)])
-def test_gemm_small_products_split_to_short_slices(gpu, M, N, K):
-    """Slices down to 32 of K fill the chip in small products: the partials of the library's split count, last
-    slices that are short or empty among them, sum to the product."""
-    g = torch.Generator().manual_seed(M + N + K)
-    A, B = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g)
-    for trans in (False, True):
-        P, splits = ops.gemm_splitk(A.to(gpu), (B.T.contiguous() if trans else B).to(gpu), trans_b=trans)
-        assert splits > 1
-        assert _rel(P.sum(0).cpu(), A.double() @ B.double()) < 2e-6
