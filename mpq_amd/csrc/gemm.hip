@@ -784,20 +784,17 @@ hipError_t splitk_reduce(const float* P, int splits, int64_t split_stride, int64
 
 bool x6_shape_ok(int64_t N, int64_t K) { return N > 0 && K > 0 && N % 128 == 0 && K % 32 == 0; }
 
-// Split K until the grid holds about two work-groups per CU (512) or a K slice would fall below 512: past that,
-// more splits do not speed the product up and every split is one more partial the epilogues read.
-// 128 x 14336 x 14336: 4 splits; 128 x 4096 x 4096: 8 splits, 24.1 us (16: 23.9).  A product too small to fill
-// one work-group per CU that way is a chain of slabs in a few work-groups: there, slices go down to 64 (one turn
-// of the LDS ring) while the grid has at most 256.  us with slices of 512 and with these: 128 x 512 x 512
-// 17.7 / 7.9, 128 x 1024 x 1024 17.7 / 8.7, 128 x 2048 x 2048 18.7 / 12.5, 128 x 3072 x 3072 25.6 / 18.3
-// (20.0 with 16 splits, 384 work-groups), 256 x 1024 x 1024 24.4 / 11.8, 256 x 2048 x 2048 25.3 / 18.7.
+// Split K until the grid holds about two work-groups per CU (512) or a K slice would fall below
+// 32 slabs (512): more splits do not speed the product up and every split is one more partial the
+// epilogues read.  128 x 14336 x 14336: 4 splits, 0.292 ms per product and 8.7 us to read the
+// partials back, against 0.298 ms and 20.7 us with 16 (the down_proj layer: 2 splits 1085 ms, 4
+// splits 1053-1062 ms).  128 x 4096 x 4096: 8 splits; a 14336 x 4096 gate_proj layer takes 391 ms
+// against 414 ms with 16 splits, 451 ms with 4 and 619 ms with 2.
 int x6_choose_splits(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ((M + 127) / 128) * (N / 128);
-  auto more = [&](int64_t s) {
-    return (tiles * s <= 512 && K % (s * 32) == 0 && K / s >= 512) || (tiles * s <= 256 && K % (s * 64) == 0);
-  };
   int splits = 1;
-  while (splits < 16 && more(splits * 2)) splits *= 2;
+  while (splits < 16 && tiles * splits * 2 <= 512 && K % (splits * 2 * 32) == 0 && K / (splits * 2) >= 512)
+    splits *= 2;
   return splits;
 }
 

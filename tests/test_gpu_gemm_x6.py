@@ -186,18 +186,3 @@ def test_pair_product_non_finite_stays_in_its_row_and_column(gpu):
     bad = torch.zeros(M, N, dtype=torch.bool)
     bad[3], bad[7], bad[:, 11] = True, True, True
     assert not bool(torch.isfinite(C[bad]).any()) and torch.equal(C[~bad], C0[~bad])
-
-
-@pytest.mark.parametrize("M,N,K,splits", [(128, 128, 64, 1), (1, 128, 128, 2), (100, 384, 384, 2), (128, 1024, 1024, 16),
-                                          (256, 1152, 1152, 2), (128, 2048, 2048, 16), (256, 2048, 2048, 8)])
-def test_gemm_x6_short_slices(gpu, M, N, K, splits):
-    """K slices of 64 and up for a grid of at most 256 work-groups.  Entry-wise error relative to
-    sum_k |a_k b_k|: one rounding per MFMA step of a slice (3 products per 16 k), one per partial summed and
-    about three for the two f16 pairs and the dropped lo x lo product."""
-    g = torch.Generator().manual_seed(M + N + K)
-    A = torch.randn(M, K, generator=g) * torch.exp(2.0 * torch.randn(1, K, generator=g))
-    B = torch.randn(K, N, generator=g)
-    assert ops._lib.load().mpq_gemm_x6_split_count(M, N, K) == splits
-    C = ops.gemm_x6(A.to(gpu), ops.gemm_x6_pack_b(B.to(gpu)), N).cpu().double()
-    err = (C - A.double() @ B.double()).abs() / (A.double().abs() @ B.double().abs())
-    assert float(err.max()) <= (3 * K / (16 * splits) + splits + 3) * 2.0**-24
