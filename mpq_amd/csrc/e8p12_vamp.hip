@@ -270,7 +270,7 @@ extern "C" int mpq_e8p12_vamp_solve_ex(int64_t rows, int64_t n, const float* Wr,
   // rewrites x1), so they are queued behind the first denoiser pass before its status is read
   auto launch_lmmse_head = [&](float obs_f) -> int {
     hipLaunchKernelGGL(msg_r2_kernel, eg, eb, 0, stream, n, x1, r1, eta1, g1w, g2new, has_prev ? 1 : 0, damping,
-                       r2prev, r2, planes, rows, (int64_t)0);
+                       r2prev, r2, planes);
     MPQ_LAUNCH_CHECK();
     MPQ_HIP_TRY(prod(r2, V, false, 0, planes != nullptr));
     hipLaunchKernelGGL(lmmse_epi1_kernel, eg, eb, 0, stream, n, P, nsplit, sstride, Yu, S, g2, obs_f, x1, part,

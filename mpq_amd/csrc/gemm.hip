@@ -542,47 +542,42 @@ constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) |
 // but the n most recent loads of this wave done, i.e. the slab about to be read).  The barrier is
 // s_barrier without a fence (the fence of __syncthreads would wait for every load in flight).
 // kRagged: K slices of any number of slabs; otherwise every slice is a positive multiple of four.
-// MT: 128-row tiles per work-group, four waves each (two tiles: 512 threads, one work-group per CU; the
-// tiles share the slabs of B, so B is read once for 256 rows).
 // kStream: B is read with the non-temporal hint (it does not fit the caches anyway).
-template <int MT, bool kRagged, bool kStream>
-__global__ __launch_bounds__(kThreads* MT, 2) void gemm_x6_kernel(int64_t M, int64_t N, int64_t K,
+template <bool kRagged, bool kStream>
+__global__ __launch_bounds__(kThreads, 2) void gemm_x6_kernel(int64_t M, int64_t N, int64_t K,
                                                               const uint4* __restrict__ At,
                                                               const float* __restrict__ Bt, float* __restrict__ C,
                                                               int64_t ldc, int64_t split_stride,
                                                               int64_t k_per_split, int splits) {
   constexpr int S = 4;
-  constexpr int BOFF = 512 * MT;      // 16-byte slots of a stage: A planes, then the two halves of B
-  constexpr int STAGE = BOFF + 512;
-  constexpr int BL = 2 / MT;          // loads of B per wave
-  constexpr int LOADS = 2 + BL;       // global_load_lds per wave per slab
+  constexpr int STAGE = 512 + 512;  // 16-byte slots: A planes, then the two halves of B
+  constexpr int LOADS = 4;          // global_load_lds per wave per slab: 2 (A) + 2 (B)
   constexpr int RT = 4;             // 32-row tiles of a wave (128 x 32)
   constexpr int FAC = 16;           // chunks of A's scales kept in LDS
   __shared__ uint4 st0[STAGE];
   __shared__ uint4 st1[STAGE];
   __shared__ uint4 st2[STAGE];
   __shared__ uint4 st3[STAGE];
-  __shared__ float fac[FAC][128 * MT];
+  __shared__ float fac[FAC][128];
   auto stage = [&](int slot) -> uint4* { return slot == 0 ? st0 : slot == 1 ? st1 : slot == 2 ? st2 : st3; };
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 2, wn = wave & 3;  // this wave's row tile and 32 columns
   const unsigned utile = blockIdx.x / (unsigned)splits, ntn = (unsigned)(N / 128);  // 32-bit divisions: short
   const int split = (int)(blockIdx.x - utile * (unsigned)splits);
-  const int64_t mt = utile / ntn * MT, nt = utile % ntn;
+  const int64_t mt = utile / ntn, nt = utile % ntn;
   const int64_t KS = K / 16;
   const int nslab = (int)(k_per_split / 16);
   const int64_t ks0 = (int64_t)split * nslab;
-  // a wave moves 128 slots of its row tile of A and 64 BL slots of B; lane l adds 16 l bytes
-  const uint4* asrc = At + ((mt + wm) * KS + ks0) * 512 + wn * 128 + lane;
-  const uint4* bsrc = reinterpret_cast<const uint4*>(Bt) + (nt * KS + ks0) * 512 + wave * 64 * BL + lane;
+  // wave w moves A slots w*128 + 64 q and B slots w*128 + 64 q (q < 2); lane l adds 16 l bytes
+  const uint4* asrc = At + (mt * KS + ks0) * 512 + wave * 128 + lane;
+  const uint4* bsrc = reinterpret_cast<const uint4*>(Bt) + (nt * KS + ks0) * 512 + wave * 128 + lane;
   auto issue = [&](int s, int slot) {
     uint4* d = stage(slot);
 #pragma unroll
     for (int q = 0; q < 2; ++q)
       __builtin_amdgcn_global_load_lds(asrc + (int64_t)s * 512 + q * 64, d + wave * 128 + q * 64, 16, 0, 0);
 #pragma unroll
-    for (int q = 0; q < BL; ++q)
-      __builtin_amdgcn_global_load_lds(bsrc + (int64_t)s * 512 + q * 64, d + BOFF + wave * 64 * BL + q * 64, 16, 0,
+    for (int q = 0; q < 2; ++q)
+      __builtin_amdgcn_global_load_lds(bsrc + (int64_t)s * 512 + q * 64, d + 512 + wave * 128 + q * 64, 16, 0,
                                        kStream ? 2 : 0);
   };
   // slabs past the end of the slice are the last one again (never multiplied), so every step issues the
@@ -596,13 +591,13 @@ __global__ __launch_bounds__(kThreads* MT, 2) void gemm_x6_kernel(int64_t M, int
   float fq[FAC / 2];
 #pragma unroll
   for (int q = 0; q < FAC / 2; ++q) {
-    const int c = 2 * q + ((tid >> 7) & 1), r = wm * 128 + (tid & 127);
-    fq[q] = inv[(c0 + (c < nch ? c : nch - 1)) * Mp + r];
+    const int c = 2 * q + (tid >> 7);
+    fq[q] = inv[(c0 + (c < nch ? c : nch - 1)) * Mp + (tid & 127)];
   }
 #pragma unroll
   for (int t = 0; t < S - 1; ++t) issue(clamp_slab(t), t);
 #pragma unroll
-  for (int q = 0; q < FAC / 2; ++q) fac[2 * q + ((tid >> 7) & 1)][wm * 128 + (tid & 127)] = fq[q];
+  for (int q = 0; q < FAC / 2; ++q) fac[2 * q + (tid >> 7)][tid & 127] = fq[q];
 
   floatx16 acc[RT], total[RT];
 #pragma unroll
@@ -621,7 +616,7 @@ __global__ __launch_bounds__(kThreads* MT, 2) void gemm_x6_kernel(int64_t M, int
     for (int i = 0; i < RT; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int r = wm * 128 + i * 32 + q * 8 + rbase;
+        const int r = i * 32 + q * 8 + rbase;
         const float4 f = nch <= FAC ? *reinterpret_cast<const float4*>(&fac[c][r])
                                     : *reinterpret_cast<const float4*>(inv + (int64_t)(c0 + c) * Mp + r);
         const float fv[4] = {f.x, f.y, f.z, f.w};
@@ -639,9 +634,9 @@ __global__ __launch_bounds__(kThreads* MT, 2) void gemm_x6_kernel(int64_t M, int
 #pragma unroll
     for (int pl = 0; pl < 2; ++pl)
 #pragma unroll
-      for (int i = 0; i < RT; ++i) a[pl][i] = __builtin_bit_cast(f16x8, d[wm * 512 + pl * 256 + i * 64 + lane]);
-    const float4 x = __builtin_bit_cast(float4, d[BOFF + wn * 64 + lane]);
-    const float4 y = __builtin_bit_cast(float4, d[BOFF + 256 + wn * 64 + lane]);
+      for (int i = 0; i < RT; ++i) a[pl][i] = __builtin_bit_cast(f16x8, d[pl * 256 + i * 64 + lane]);
+    const float4 x = __builtin_bit_cast(float4, d[512 + wave * 64 + lane]);
+    const float4 y = __builtin_bit_cast(float4, d[512 + 256 + wave * 64 + lane]);
     const float m = fmaxf(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))),
                           fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
     if (__builtin_amdgcn_ballot_w64(m > blim)) {  // rare: a column outgrew its scale
@@ -699,12 +694,12 @@ __global__ __launch_bounds__(kThreads* MT, 2) void gemm_x6_kernel(int64_t M, int
 
   const int col = lane & 31;
   float* Cs = C + (int64_t)split * split_stride;
-  const int64_t gn = nt * 128 + wn * 32 + col;
+  const int64_t gn = nt * 128 + wave * 32 + col;
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const int64_t gm = (mt + wm) * 128 + i * 32 + (v >> 2) * 8 + rbase + (v & 3);
+      const int64_t gm = mt * 128 + i * 32 + (v >> 2) * 8 + rbase + (v & 3);
       if (gm < M) Cs[gm * ldc + gn] = total[i][v];
     }
 }
@@ -826,23 +821,16 @@ hipError_t x6_gemm_partials(const void* At, const float* Bt, int64_t M, int64_t 
                             int64_t split_stride, int splits, hipStream_t stream) {
   const int64_t kps = K / splits;
   if (!x6_shape_ok(N, K) || splits < 1 || K % splits != 0 || kps % 32 != 0) return hipErrorInvalidValue;
-  // pairs of row tiles share B where there are any: 256 x 14336 x 14336 410 -> 346 us, 4096 x 14336 x 14336
-  // 5.56 -> 4.95 ms, 4096 x 4096 x 4096 420 -> 390 us
-  const int64_t mtiles = (M + 127) / 128;
-  const int mt = mtiles % 2 == 0 ? 2 : 1;
-  const int64_t blocks = mtiles / mt * (N / 128) * splits;
+  const int64_t blocks = ((M + 127) / 128) * (N / 128) * splits;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
   // An operator larger than the 256 MB last-level cache is gone before the next product reads it, and only
   // pushes the other operands out: 128 x 14336 x 14336 takes 199 us with the hint and 210 without; 4096 x 4096
   // (64 MB, which stays cached between products) 31.1 with and 28.2 without.
   const bool ragged = (kps / 16) % 4 != 0, big = K * N * 4 >= ((int64_t)256 << 20);
-  const auto kernel =
-      mt == 2 ? (ragged ? (big ? gemm_x6_kernel<2, true, true> : gemm_x6_kernel<2, true, false>)
-                        : (big ? gemm_x6_kernel<2, false, true> : gemm_x6_kernel<2, false, false>))
-              : (ragged ? (big ? gemm_x6_kernel<1, true, true> : gemm_x6_kernel<1, true, false>)
-                        : (big ? gemm_x6_kernel<1, false, true> : gemm_x6_kernel<1, false, false>));
-  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kThreads * mt), 0, stream, M, N, K,
-                     static_cast<const uint4*>(At), Bt, C, ldc, split_stride, kps, splits);
+  const auto kernel = ragged ? (big ? gemm_x6_kernel<true, true> : gemm_x6_kernel<true, false>)
+                             : (big ? gemm_x6_kernel<false, true> : gemm_x6_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, M, N, K, static_cast<const uint4*>(At),
+                     Bt, C, ldc, split_stride, kps, splits);
   return hipGetLastError();
 }
 

@@ -181,7 +181,7 @@ __global__ __launch_bounds__(kEW) void epi2_denoise_kernel(
     const float* __restrict__ eta2, const float* __restrict__ g2, const float* __restrict__ g1new, float damping,
     float* __restrict__ r1, const float* __restrict__ gamma, const float* __restrict__ W, int64_t ldw,
     const float* __restrict__ scale, const float* __restrict__ zero, int64_t G, int64_t gs, int maxq, float tau,
-    uint8_t* __restrict__ q_out, float* __restrict__ x_out, uint4* __restrict__ planes, int64_t plane_rows) {
+    uint8_t* __restrict__ q_out, float* __restrict__ x_out, uint4* __restrict__ planes) {
   static_assert(HMODE == kHardMap || HMODE == kHardRoundMean, "hard decision modes");
   __shared__ float red[kEW / 64];
   __shared__ __attribute__((aligned(16))) float s_v[kChunk];
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(kEW) void epi2_denoise_kernel(
   }
   if (planes) {
     __syncthreads();
-    chunk_planes(planes, plane_rows, n, b, s_v, red);
+    chunk_planes(planes, gridDim.y, n, b, s_v, red);
   }
 }
 
@@ -246,7 +246,6 @@ struct Workspace {
   int splits;      // of the active product path
   int splits_f32;
   int splits_x6;   // 0 if the shape has no x6 path
-  int splits_pair;  // of the x6 product of pair_rows rows
   int bn;
   const float* packed;  // rank-space operator of the x6 path, or null (fp32 path)
 };
@@ -254,20 +253,9 @@ struct Workspace {
 inline int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 struct Sizes {
-  int64_t rows, n, nchunks, splits, splits_x6, splits_pair, bn;
+  int64_t rows, n, nchunks, splits, splits_x6, bn;
   int64_t bytes;
 };
-
-// Left operand of the x6 product that takes an iteration's hard state and the next one's r2 message at
-// once: the hard state's rows from row 0, the message's from row pair_row0.
-inline int64_t pair_row0(int64_t rows) { return align_up(rows, 128); }
-inline int64_t pair_rows(int64_t rows) { return pair_row0(rows) + rows; }
-
-// Floats of the split-K partials of any of the solver's products.
-inline int64_t partial_floats(const Sizes& s) {
-  const int64_t one = std::max(s.splits, s.splits_x6) * align_up(s.rows * s.n, 64);
-  return std::max(one, s.splits_pair * align_up(pair_rows(s.rows) * s.n, 64));
-}
 
 Sizes plan(int64_t rows, int64_t n) {
   Sizes s;
@@ -277,13 +265,12 @@ Sizes plan(int64_t rows, int64_t n) {
   int bn = 128;
   s.splits = choose_splits(rows, n, n, (int64_t)1 << 62, &bn);
   s.splits_x6 = x6_shape_ok(n, n) ? x6_choose_splits(rows, n, n) : 0;
-  s.splits_pair = s.splits_x6 ? x6_choose_splits(pair_rows(rows), n, n) : 0;
   s.bn = bn;
   const int64_t mat = align_up(rows * n, 64) * 4;
   int64_t bytes = 0;
   bytes += 8 * mat;                                   // Yu r1 r2 r2prev x1 xs prod_cur prod_best
-  bytes += partial_floats(s) * 4;                     // P
-  bytes += s.splits_x6 ? align_up(x6_packed_a_bytes(pair_rows(rows), n), 256) : 0;  // Ap
+  bytes += std::max(s.splits, s.splits_x6) * mat;     // P
+  bytes += s.splits_x6 ? align_up(x6_packed_a_bytes(rows, n), 256) : 0;  // Ap
   bytes += align_up(32 * rows, 64) * 4;               // row arrays
   bytes += align_up(3 * rows * s.nchunks, 64) * 4;    // chunk partials
   bytes += 2 * align_up(rows * n, 256);               // q_cur q_best
@@ -304,9 +291,9 @@ Workspace carve(void* base, const Sizes& s) {
   w.xs = (float*)p; p += mat;
   w.prod_cur = (float*)p; p += mat;
   w.prod_best = (float*)p; p += mat;
-  w.P = (float*)p; p += partial_floats(s) * 4;
+  w.P = (float*)p; p += std::max(s.splits, s.splits_x6) * mat;
   w.Ap = s.splits_x6 ? (void*)p : nullptr;
-  p += s.splits_x6 ? align_up(x6_packed_a_bytes(pair_rows(s.rows), s.n), 256) : 0;
+  p += s.splits_x6 ? align_up(x6_packed_a_bytes(s.rows, s.n), 256) : 0;
   w.rowbuf = (float*)p; p += align_up(32 * s.rows, 64) * 4;
   w.part = (float*)p; p += align_up(3 * s.rows * s.nchunks, 64) * 4;
   w.q_cur = (uint8_t*)p; p += align_up(s.rows * s.n, 256);
@@ -314,7 +301,6 @@ Workspace carve(void* base, const Sizes& s) {
   w.status = (VampStatus*)p;
   w.splits = w.splits_f32 = (int)s.splits;
   w.splits_x6 = (int)s.splits_x6;
-  w.splits_pair = (int)s.splits_pair;
   w.bn = (int)s.bn;
   w.packed = nullptr;
   return w;
@@ -404,27 +390,11 @@ int uniform_vamp_solve(const UniformProblem& pr, const float* Vs, const MpqUnifo
   const float tau = cfg.prior_tau;
   int rc;
 
-  // A decision's rank-space error from its product with the rank-space operator, whose partials are in
-  // w.P: with a packed operator the product is x V, and x Vs = (x V) diag(S).
-  const float* const xS = w.packed ? pr.S : nullptr;
-  const RankOperand xop = w.packed ? kOpV : kOpVs;
-  auto launch_err = [&](int splits, int64_t stride) -> int {
-    hipLaunchKernelGGL(err_epi_kernel, eg, eb, 0, stream, n, w.P, splits, stride, Yu, w.part,
-                       pr.xprod_out ? w.prod_cur : nullptr, xS);
-    MPQ_LAUNCH_CHECK();
-    return kOk;
-  };
-  // its row kernel, which publishes the status (hard_seq)
-  auto publish_err = [&]() -> int {
-    hard_seq = ++mb->seq;
-    hipLaunchKernelGGL(rows_err_kernel, dim3(1), eb, 0, stream, rows, nchunks, w.part, err_cur, w.status, mb->dev(hard_seq),
-                       hard_seq);
-    MPQ_LAUNCH_CHECK();
-    return kOk;
-  };
-  // hard decision of (r, g) -> q_cur, xs, and its error -> err_cur, status.err_mean
-  auto hard_state = [&](const float* r, const float* g) -> int {
-    if (cfg.final_decision == 1) {
+  // hard state + rank-space error of the decision for (r1, g1) -> q_cur, err_cur, status.err_mean
+  // (decided: the denoiser's decision is already in q_cur / xs / planes, from epi2_denoise_kernel)
+  auto hard_state = [&](const float* r, const float* g, bool decided) -> int {
+    if (decided) {
+    } else if (cfg.final_decision == 1) {
       hipLaunchKernelGGL(uniform_denoise_kernel<kHardRoundMean>, eg, eb, 0, stream, r, g, pr.W, pr.ldw,
                          pr.scale, pr.zero, G, pr.group_size, n, pr.maxq, tau, nullptr, nullptr,
                          w.q_cur, w.xs, planes);
@@ -434,9 +404,15 @@ int uniform_vamp_solve(const UniformProblem& pr, const float* Vs, const MpqUnifo
                          w.q_cur, w.xs, planes);
     }
     MPQ_LAUNCH_CHECK();
-    MPQ_HIP_TRY(product(w, w.xs, Vs, false, xop, rows, n, stream, planes != nullptr));
-    int e = launch_err(w.splits, sstride);
-    return e != kOk ? e : publish_err();
+    MPQ_HIP_TRY(product(w, w.xs, Vs, false, kOpVs, rows, n, stream, planes != nullptr));
+    hipLaunchKernelGGL(err_epi_kernel, eg, eb, 0, stream, n, w.P, w.splits, sstride, Yu, w.part,
+                       pr.xprod_out ? w.prod_cur : nullptr);
+    // the row kernel publishes the status (hard_seq) for the wait that follows every hard state
+    hard_seq = ++mb->seq;
+    hipLaunchKernelGGL(rows_err_kernel, dim3(1), eb, 0, stream, rows, nchunks, w.part, err_cur, w.status, mb->dev(hard_seq),
+                       hard_seq);
+    MPQ_LAUNCH_CHECK();
+    return kOk;
   };
 
   // ---- setup ----------------------------------------------------------
@@ -492,7 +468,7 @@ int uniform_vamp_solve(const UniformProblem& pr, const float* Vs, const MpqUnifo
     MPQ_HIP_TRY(copy_rows(w.r1, n * 4, src, pr.ldw * 4, rows, n * 4, stream));
   }
   // initial hard state = best
-  if ((rc = hard_state(w.r1, g1)) != kOk) return rc;
+  if ((rc = hard_state(w.r1, g1, false)) != kOk) return rc;
   if ((rc = wait_status(mb, hard_seq, hs, stream)) != kOk) return rc;
   double best_err_mean = (double)hs->err_mean;
   std::swap(w.q_cur, w.q_best);
@@ -521,37 +497,22 @@ int uniform_vamp_solve(const UniformProblem& pr, const float* Vs, const MpqUnifo
                        has_prev ? 1 : 0, damping, g2prev, a1raw, a1, eta1, g2new, g2, w.status, mb->dev(seq), seq);
     return seq;
   };
-  // r2 message of (x1, r1); `planes` receives it as rows row0 .. of an operand of prows rows
-  auto launch_r2 = [&](int64_t prows, int64_t row0) -> int {
-    hipLaunchKernelGGL(msg_r2_kernel, eg, eb, 0, stream, n, w.x1, w.r1, eta1, g1w, g2new, has_prev ? 1 : 0, damping,
-                       w.r2prev, w.r2, planes, prows, row0);
-    MPQ_LAUNCH_CHECK();
-    return kOk;
-  };
-  // LMMSE part 1 from the partials of r2 V (obs as used by this iteration)
-  auto launch_epi1 = [&](const float* P, int splits, int64_t stride, float obs_f) -> int {
-    hipLaunchKernelGGL(lmmse_epi1_kernel, eg, eb, 0, stream, n, P, splits, stride, Yu, pr.S, g2, obs_f, w.x1, w.part,
-                       planes);
-    MPQ_LAUNCH_CHECK();
-    return kOk;
-  };
-  // The LMMSE head of an iteration: message, product, part 1 (the latter two here).  It writes only the
+  // r2 message and the first LMMSE product (obs as used by this iteration).  They write only the
   // message, the product's partials, the LMMSE mean (in x1) and its row partials, which a gamma retry
-  // recomputes from scratch (the retried denoiser rewrites x1), so it is queued behind the first denoiser pass
-  // before that pass's status is read, and the GPU has work while the host waits; after a retry (g1w rescaled)
-  // it runs again from the retried pass.
+  // recomputes from scratch (the retried denoiser rewrites x1), so the loop queues them behind the
+  // first denoiser pass before that pass's status is read, and the GPU has work while the host
+  // waits; after a retry (g1w rescaled) they run again from the retried pass.
   auto launch_lmmse_head = [&](float obs_f) -> int {
+    hipLaunchKernelGGL(msg_r2_kernel, eg, eb, 0, stream, n, w.x1, w.r1, eta1, g1w, g2new,
+                       has_prev ? 1 : 0, damping, w.r2prev, w.r2, planes);
+    MPQ_LAUNCH_CHECK();
     MPQ_HIP_TRY(product(w, w.r2, pr.V, false, kOpV, rows, n, stream, planes != nullptr));
-    return launch_epi1(w.P, w.splits, sstride, obs_f);
+    hipLaunchKernelGGL(lmmse_epi1_kernel, eg, eb, 0, stream, n, w.P, w.splits, sstride, Yu, pr.S, g2,
+                       obs_f, w.x1, w.part, planes);
+    MPQ_LAUNCH_CHECK();
+    return kOk;
   };
-  // The loop queues an iteration's error evaluation together with the next iteration's first denoiser pass
-  // and message; with a packed operator, with its whole LMMSE head: both products take the operator V, so with a packed operator they are one product of
-  // pair_rows rows that reads V once (128-row blocks: 346 us at n = 14336
-  // against 2 x 202, 33 against 2 x 25 at 4096).  The next head's part 1 needs the updated
-  // observation precision, whose statistic the LMMSE row kernel publishes on its own well before.  After a
-  // stop the head's results are never read.
-  const int64_t prow0 = pair_row0(rows), prows = pair_rows(rows), pstride = align_up(prows * n, 64);
-  unsigned ahead_seq = 0;  // status of the iteration's first denoiser pass, queued with its head by the one before
+  unsigned ahead_seq = 0;  // the iteration's first denoiser pass, launched at the end of the one before
   for (int it = 0; it < iters; ++it) {
     // ---- denoiser with gamma retries (mpq/solver.py:559-596), from g1w = g1
     if (ahead_seq == 0) {
@@ -559,23 +520,17 @@ int uniform_vamp_solve(const UniformProblem& pr, const float* Vs, const MpqUnifo
       g1w_current = true;
     }
     const float obs_f = (float)obs;
-    // the LMMSE head of the pass whose status is read last; the one before queued it with that pass, or only
-    // its message
-    bool head_queued = ahead_seq != 0 && w.packed;
-    if (ahead_seq != 0 && !w.packed) {
-      if ((rc = launch_lmmse_head(obs_f)) != kOk) return rc;
-      head_queued = true;
-    }
+    bool head_queued = false;  // the LMMSE head of the pass whose status is read last
     for (int attempt = 0; attempt <= retry_steps; ++attempt) {
       unsigned a1_seq = ahead_seq;
       ahead_seq = 0;
       if (a1_seq == 0) {
         a1_seq = launch_alpha1();
         MPQ_LAUNCH_CHECK();
-        if (attempt == 0) {
-          if ((rc = launch_r2(rows, 0)) != kOk || (rc = launch_lmmse_head(obs_f)) != kOk) return rc;
-          head_queued = true;
-        }
+      }
+      if (attempt == 0) {
+        if ((rc = launch_lmmse_head(obs_f)) != kOk) return rc;
+        head_queued = true;
       }
       if ((rc = wait_status(mb, a1_seq, hs, stream)) != kOk) return rc;
       if (hs->a1_invalid == 0) break;
@@ -599,49 +554,37 @@ int uniform_vamp_solve(const UniformProblem& pr, const float* Vs, const MpqUnifo
     }
     const float a1_mean_it = hs->a1_mean;
     // ---- LMMSE
-    if (!head_queued && ((rc = launch_r2(rows, 0)) != kOk || (rc = launch_lmmse_head(obs_f)) != kOk)) return rc;
-    const unsigned em_seq = ++mb->seq;
+    if (!head_queued && (rc = launch_lmmse_head(obs_f)) != kOk) return rc;
     hipLaunchKernelGGL(rows_lmmse_kernel, dim3(1), eb, 0, stream, rows, n, n, nchunks, w.part, g2, damping,
-                       eta2, g1new, g1, g1w, w.status, mb->dev(em_seq), em_seq);
+                       eta2, g1new, g1, g1w, w.status);
     MPQ_LAUNCH_CHECK();
-    g1w_current = true;
     MPQ_HIP_TRY(product(w, w.x1, pr.V, true, kOpVt, rows, n, stream, planes != nullptr));
-    // ---- r1 message and the hard decision of the new (r1, g1)
-    const bool next = it + 1 < iters, paired = next && w.packed;
-    const int64_t xrows = paired ? prows : rows;
+    // ---- r1 message and the hard state of the new (r1, g1)
     if (cfg.final_decision == 1) {
       hipLaunchKernelGGL(epi2_denoise_kernel<kHardRoundMean>, eg, eb, 0, stream, n, w.P, w.splits, sstride, w.r2,
                          eta2, g2, g1new, damping, w.r1, g1, pr.W, pr.ldw, pr.scale, pr.zero, G, pr.group_size,
-                         pr.maxq, tau, w.q_cur, w.xs, planes, xrows);
+                         pr.maxq, tau, w.q_cur, w.xs, planes);
     } else {
       hipLaunchKernelGGL(epi2_denoise_kernel<kHardMap>, eg, eb, 0, stream, n, w.P, w.splits, sstride, w.r2, eta2,
                          g2, g1new, damping, w.r1, g1, pr.W, pr.ldw, pr.scale, pr.zero, G, pr.group_size, pr.maxq,
-                         tau, w.q_cur, w.xs, planes, xrows);
+                         tau, w.q_cur, w.xs, planes);
     }
     MPQ_LAUNCH_CHECK();
+    if ((rc = hard_state(w.r1, g1, true)) != kOk) return rc;
     std::swap(w.r2, w.r2prev);  // r2_prev <- r2
     std::swap(g2, g2prev);      // gamma2_prev <- gamma2
     has_prev = true;
-    // ---- its rank-space error; the next iteration's first denoiser pass and message read only device
-    // state (r1, gamma1, and gamma2 of this iteration)
-    if (next) {
+    // The next iteration's first denoiser pass reads only device state (r1, gamma1, and gamma2 of
+    // this iteration), so it is queued before this iteration's status is read and the GPU works
+    // through the host's EM and stopping decision.  After a stop its results are never read.
+    if (it + 1 < iters) {
+      if (!g1w_current) MPQ_HIP_TRY(copy_rows(g1w, 0, g1, 0, 1, rows * 4, stream));
+      g1w_current = true;
       ahead_seq = launch_alpha1();
       MPQ_LAUNCH_CHECK();
-      if ((rc = launch_r2(prows, prow0)) != kOk) return rc;
     }
-    if (paired) {
-      MPQ_HIP_TRY(x6_gemm_partials(w.Ap, w.packed + (int64_t)kOpV * n * n, prows, n, n, w.P, n, pstride, w.splits_pair,
-                                   stream));
-      if ((rc = launch_err(w.splits_pair, pstride)) != kOk) return rc;
-    } else {
-      MPQ_HIP_TRY(product(w, w.xs, Vs, false, xop, rows, n, stream, planes != nullptr));
-      if ((rc = launch_err(w.splits, sstride)) != kOk) return rc;
-    }
-    // read before anything publishes two statuses later (the mailbox has two slots)
-    if ((rc = wait_status(mb, em_seq, hs, stream)) != kOk) return rc;
-    if ((rc = publish_err()) != kOk) return rc;
+    if ((rc = wait_status(mb, hard_seq, hs, stream)) != kOk) return rc;
     a2_clip += hs->a2_clip;
-    a2_sum += hs->a2_mean;
     // EM update of the observation precision (mpq/linear.py:59-82), in double like the reference
     if (em_active) {
       float den = hs->em_mean < 1e-12f ? 1e-12f : hs->em_mean;
@@ -657,11 +600,8 @@ int uniform_vamp_solve(const UniformProblem& pr, const float* Vs, const MpqUnifo
     }
     obs_sum += obs;
     a1_sum += a1_mean_it;
+    a2_sum += hs->a2_mean;
     ++n_logged;
-    if (paired) {  // the rest of the next iteration's head
-      if ((rc = launch_epi1(w.P + prow0 * n, w.splits_pair, pstride, (float)obs)) != kOk) return rc;
-    }
-    if ((rc = wait_status(mb, hard_seq, hs, stream)) != kOk) return rc;
     // best iterate (mpq/solver.py:678-699)
     const double cur = (double)hs->err_mean;
     const double tol = std::max(1e-10, std::fabs(best_err_mean) * 1e-8);
@@ -679,9 +619,12 @@ int uniform_vamp_solve(const UniformProblem& pr, const float* Vs, const MpqUnifo
     }
   }
 
-  // A stop leaves the next iteration's head queued; its denoiser status was published before the error
-  // status that was waited for, so no publish to the mailbox is outstanding when this call returns (a
-  // later call may run on another stream).
+  // a stop leaves the look-ahead pass queued: wait for its status, so that no publish to the
+  // mailbox is outstanding when this call returns (a later call may run on another stream)
+  if (ahead_seq != 0) {
+    VampStatus unused;
+    if ((rc = wait_status(mb, ahead_seq, &unused, stream)) != kOk) return rc;
+  }
   // ---- outputs
   MPQ_HIP_TRY(copy_rows(q_out, 0, w.q_best, 0, 1, rows * n, stream));
   if (err_out) MPQ_HIP_TRY(copy_rows(err_out, 0, err_best, 0, 1, rows * 4, stream));

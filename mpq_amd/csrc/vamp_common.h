@@ -58,9 +58,9 @@ __device__ __forceinline__ void publish_to(const VampStatus* st, StatusMailbox* 
 
 static_assert(kChunk == kPairChunk && kEW == 256, "a work-group's columns are one scale group of the packed operand");
 
-// Pair planes of this work-group's column chunk, staged in s_v (column blockIdx.x * kChunk + i at
-// s_v[i]), at their place in the packed left operand At of the next x6 product (n % 16 == 0): row b of
-// `rows`.  The producing kernels write them so the product needs no packing launch.
+// Pair planes of this work-group's column chunk of row b (of `rows`), staged in s_v (column
+// blockIdx.x * kChunk + i at s_v[i]), at their place in the packed left operand At of the next x6
+// product (n % 16 == 0).  The producing kernels write them so the product needs no packing launch.
 // All threads call it; `red`: 4 floats of LDS.
 __device__ __forceinline__ void chunk_planes(uint4* __restrict__ At, int64_t rows, int64_t n, int64_t b,
                                              const float* s_v, float* red) {
@@ -227,16 +227,14 @@ __global__ void rows_retry_kernel(int64_t rows, const float* __restrict__ alpha1
   }
 }
 
-// r2 message (mpq/solver.py:605-612).  `planes`: packed left operand of plane_rows rows that receives the
-// message as rows plane_row0 + b.
+// r2 message (mpq/solver.py:605-612).
 __global__ __launch_bounds__(kEW) void msg_r2_kernel(int64_t n, const float* __restrict__ x1,
                                                      const float* __restrict__ r1,
                                                      const float* __restrict__ eta1,
                                                      const float* __restrict__ g1w,
                                                      const float* __restrict__ g2new, int has_prev,
                                                      float damping, const float* __restrict__ r2prev,
-                                                     float* __restrict__ r2, uint4* __restrict__ planes,
-                                                     int64_t plane_rows, int64_t plane_row0) {
+                                                     float* __restrict__ r2, uint4* __restrict__ planes) {
   __shared__ float red[kEW / 64];
   __shared__ __attribute__((aligned(16))) float s_v[kChunk];
   const int64_t b = blockIdx.y;
@@ -255,7 +253,7 @@ __global__ __launch_bounds__(kEW) void msg_r2_kernel(int64_t n, const float* __r
   }
   if (planes) {  // uniform
     __syncthreads();
-    chunk_planes(planes, plane_rows, n, plane_row0 + b, s_v, red);
+    chunk_planes(planes, gridDim.y, n, b, s_v, red);
   }
 }
 
@@ -389,13 +387,11 @@ __global__ __launch_bounds__(kEW) void lmmse_epi2_kernel(
 }
 
 // Rank-space error partials (mpq/linear.py:94): sum_j (Yu - sum_s P[s])^2.
-// prod (optional, rows x n) receives the summed product x Vs; with S the partials are those of x V, and
-// x Vs = (x V) diag(S).
+// prod (optional, rows x n) receives the summed product x Vs.
 __global__ __launch_bounds__(kEW) void err_epi_kernel(int64_t n, const float* __restrict__ P,
                                                       int splits, int64_t split_stride,
                                                       const float* __restrict__ Yu,
-                                                      float* __restrict__ part, float* __restrict__ prod,
-                                                      const float* __restrict__ S = nullptr) {
+                                                      float* __restrict__ part, float* __restrict__ prod) {
   __shared__ float red[kEW / 64];
   const int64_t b = blockIdx.y;
   float acc = 0.f;
@@ -404,8 +400,7 @@ __global__ __launch_bounds__(kEW) void err_epi_kernel(int64_t n, const float* __
     const int64_t j = (int64_t)blockIdx.x * kChunk + e * kEW + threadIdx.x;
     if (j >= n) continue;
     const int64_t o = b * n + j;
-    float v = sum_splits(P, splits, split_stride, o);
-    if (S) v *= S[j];
+    const float v = sum_splits(P, splits, split_stride, o);
     if (prod) prod[o] = v;
     const float d = Yu[o] - v;
     acc += d * d;
