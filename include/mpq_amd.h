@@ -160,8 +160,8 @@ int mpq_e8p12_vamp_solve(int64_t rows, int64_t n, const float* Wr, const float* 
 
 /*
  * mpq_e8p12_vamp_solve with the packed rank-space operator of mpq_rankspace_pack (`packed`,
- * nullable): the solver's products then run as x6 products on the 16-bit matrix cores
- * (fp32 accuracy).  Same products as the reference's solver (mpq/solver.py:853-1138).
+ * nullable): the solver's products then run as x6 products on the bf16 matrix cores (fp32
+ * accuracy).  Same products as the reference's solver (mpq/solver.py:853-1138).
  */
 int mpq_e8p12_vamp_solve_ex(int64_t rows, int64_t n, const float* Wr, const float* hat_init,
                             const float* V, const float* S, const float* Vs, const float* prior_scale,
@@ -247,14 +247,13 @@ int mpq_gemm_f32_splitk(int64_t M, int64_t N, int64_t K, const float* A, int64_t
                         int64_t ldb, int trans_b, float* partials, int splits, mpq_stream_t stream);
 
 /*
- * fp32 products on the 16-bit matrix cores ("x6"): each operand is held as a pair of f16 planes,
- * scaled by powers of two per row (A) and per column (B), and three plane products are accumulated in fp32
- * (v_mfma_f32_32x32x16_f16), which keeps the accuracy of an fp32 product (representation 2^-23 per
- * operand, the dropped low x low product below 2^-22 |a||b| per multiply) at 16/3 the matrix-core rate of
- * v_mfma_f32_32x32x2_f32.  (The name dates from six products of three bf16 planes.)
+ * fp32 products on the bf16 matrix cores ("x6"): each operand is split exactly into three bf16
+ * planes and the six plane products of order >= 2^-16 |a||b| are accumulated in fp32
+ * (v_mfma_f32_32x32x16_bf16), which keeps the accuracy of an fp32 product (the dropped terms are
+ * below ~2^-22.4 |a||b| per multiply) at 8/3 the matrix-core rate of v_mfma_f32_32x32x2_f32.
  * The large operand op(B) (K x N, N % 128 == 0, K % 32 == 0) is packed once into fragment-ordered
- * tiles (K * N floats, mpq_gemm_x6_pack_b; split as it is read); mpq_gemm_x6 then forms C = A op(B) for
- * any M, splitting and packing A in `workspace` (mpq_gemm_x6_workspace_size bytes) and reducing split-K partials in
+ * tiles (K * N floats, mpq_gemm_x6_pack_b); mpq_gemm_x6 then forms C = A op(B) for any M, splitting
+ * and packing A in `workspace` (mpq_gemm_x6_workspace_size bytes) and reducing split-K partials in
  * a fixed order.  Same products as mpq_gemm_f32 (no reference counterpart beyond those matmuls).
  */
 int mpq_gemm_x6_pack_b(int64_t K, int64_t N, const float* B, int64_t ldb, int trans_b, float* packed,
@@ -668,7 +667,7 @@ int mpq_uniform_cd_sweeps_noalloc(int64_t rows, int64_t n, int maxq, int64_t blo
  * that product (the reference recomputes it, mpq/solver.py:283-290).  With S (n singular values,
  * Vs = V diag(S)) and the packed rank-space operator (mpq_rankspace_pack; both optional, n % 128
  * == 0) its two full products (rhs = residual Vs^T, final x Vs; mpq/solver.py:291-330) run as
- * fp32-accurate f16-pair products on the matrix cores.
+ * fp32-accurate bf16-plane products on the matrix cores.
  */
 int mpq_uniform_cd_polish_ex(int64_t rows, int64_t n, int maxq, int64_t block_rows, int sweeps,
                              float accept_tol, const float* W, int64_t ldw, const float* Yu,

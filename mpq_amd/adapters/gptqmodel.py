@@ -50,7 +50,7 @@ class GPTQAdapterConfig:
     rotation_seed: int = 0
     auto_block_rows: bool = False
     eigen_cache: bool = True  # reuse the decomposition of an identical Hessian (q/k/v, gate/up)
-    # rank-space products as fp32-accurate f16-pair products on the matrix cores (ops.gemm_x6)
+    # rank-space products as fp32-accurate bf16-plane products on the matrix cores (ops.gemm_x6)
     # when cols % 128 == 0 and cols >= ops.X6_MIN_N; False keeps every product on the fp32 MFMA kernel
     x6_products: bool = True
 
@@ -271,7 +271,7 @@ def run_mpq_quantization(
     # Rank-space targets W Vs and the RTN decision's x_rtn Vs, formed once for all rows (the
     # reference forms them per row block inside the solver, mpq/solver.py:467-480); the row blocks
     # and the polish take slices, and each block returns its best decision's x Vs for the polish.
-    # The rank-space operator packed once per linear for the f16-pair products (None: fp32 path).
+    # The rank-space operator packed once per linear for the bf16-plane products (None: fp32 path).
     packed = ops.rankspace_pack(V, Vs) if bool(adapter_cfg.x6_products) and cols >= ops.X6_MIN_N else None
     if packed is not None:
         Vs_packed = packed[2 * cols * cols:]

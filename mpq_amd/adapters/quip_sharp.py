@@ -42,7 +42,7 @@ class QuipAdapterConfig:
     block_rows: int = 128
     jitter_base: float = 1e-6
     eigen_floor_scale: float = 1e-6
-    # rank-space products as fp32-accurate f16-pair products on the matrix cores (ops.gemm_x6)
+    # rank-space products as fp32-accurate bf16-plane products on the matrix cores (ops.gemm_x6)
     # when n % 128 == 0 and n >= ops.X6_MIN_N; False keeps every product on the fp32 MFMA kernel
     x6_products: bool = True
 
@@ -234,7 +234,7 @@ def mpq_refine_codebook(
 
     block_rows = _resolve_block_rows(m, int(getattr(args, "mpq_block_rows", adapter_cfg.block_rows)
                                             or adapter_cfg.block_rows))
-    # the rank-space operator packed once for the f16-pair products (None: fp32 path)
+    # the rank-space operator packed once for the bf16-plane products (None: fp32 path)
     packed = (ops.rankspace_pack(V, Vs) if bool(getattr(adapter_cfg, "x6_products", True)) and n >= ops.X6_MIN_N
               else None)
     requested_obs = float(getattr(args, "mpq_obs_precision", 0.0) or 0.0)

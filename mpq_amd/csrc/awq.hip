@@ -179,11 +179,10 @@ __global__ void loss_kernel(int64_t rows, const float* __restrict__ rowq, float*
 namespace mpq {
 namespace {
 
-// The search's workspace.  The 20 products D H run as x6 products on H packed once (f16 matrix cores) where
+// The search's workspace.  The 20 products D H run as x6 products on H packed once (bf16 matrix cores) where
 // the shape has them; else, and for problems so small that the launches are what counts, on the fp32 kernel.
-// 4096 x 4096, per ratio: 1.21 ms (fp32 product) -> 0.41 (x6) + 0.04 (packing D); below n = 1024 the extra
-// launches cost more than the product gains (4096 x 512, the whole search: 1.50 ms with x6, 1.20 without; 2475 x
-// 384: 1.18 / 0.94).
+// 4096 x 4096, the whole search: 23.8 ms with fp32 products, 14.9 with x6; below n = 1024 the extra
+// launches cost more than the product gains (4096 x 512: 1.27 ms with x6, 1.19 without; 2048 x 640: 1.15 / 1.12).
 struct AwqPlan {
   bool x6;
   int splits, bn;

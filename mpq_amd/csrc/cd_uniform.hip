@@ -376,7 +376,7 @@ struct CdPlan {
   int64_t rows, n, nblocks, nchunks;
   int splits, bn;
   int splits_x6;    // split count of the x6 products (0: shape not supported)
-  int64_t ap_bytes;  // packed f16 pairs of their left operand
+  int64_t ap_bytes;  // packed bf16 planes of their left operand
   int64_t bytes;
 };
 

@@ -39,7 +39,7 @@ struct E8Plan {
   int64_t rows, n, nb, nchunks;
   int splits, bn;
   int splits_x6;     // 0 if the shape has no x6 path
-  int64_t ap_bytes;  // packed f16 pairs of a product's left operand (x6 path)
+  int64_t ap_bytes;  // packed bf16 planes of a product's left operand (x6 path)
   int64_t bytes;
 };
 
@@ -165,7 +165,7 @@ extern "C" int mpq_e8p12_vamp_solve_ex(int64_t rows, int64_t n, const float* Wr,
   HostMailbox* mb = host_mailbox();
   MPQ_CHECK_ARG(mb != nullptr, "E8P12 VAMP: mapped status mailbox unavailable");
   auto sync_status = [&]() -> int { return read_status(mb, status, hs, stream); };
-  // rank-space products: on the packed operator (x6, f16 matrix cores) when given, else fp32 MFMA;
+  // rank-space products: on the packed operator (x6, bf16 matrix cores) when given, else fp32 MFMA;
   // `op` indexes the packed operator (0: V for r V, 1: V for x V^T, 2: Vs for x Vs)
   const bool x6 = packed != nullptr && pl.splits_x6 > 0;
   const int nsplit = x6 ? pl.splits_x6 : pl.splits;

@@ -55,8 +55,8 @@ hipError_t gemm_lower(const float* A, int64_t lda, const float* B, int64_t ldb, 
                       int64_t ldc, int64_t M, int64_t K, float alpha, float beta, int upper_band,
                       hipStream_t stream);
 
-// fp32 products on the f16 matrix cores (each operand a pair of scaled f16 planes, three plane products;
-// accuracy of an fp32 product, see gemm.hip).  B is packed once into fp32 tiles of
+// fp32 products on the bf16 matrix cores (each operand split exactly into three bf16 planes, six
+// plane products; accuracy of an fp32 product, see gemm.hip).  B is packed once into fp32 tiles of
 // 128 columns x 16 k (K * N floats); A is split and packed per product (x6_packed_a_bytes).
 // Shapes: N % 128 == 0, K % 32 == 0; any M (rows past M are zero in the packed A).
 bool x6_shape_ok(int64_t N, int64_t K);

@@ -14,7 +14,7 @@
 // gemm_f32_full_kernel: no bounds checks and two K slabs of global loads in flight;
 // ragged or gathered products run gemm_f32_kernel with one slab of register prefetch.
 #include "gemm.h"
-#include "f16_pair.h"
+#include "x6_split.h"
 
 namespace mpq {
 namespace {
@@ -457,33 +457,32 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_full_kernel(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// fp32 product on the 16-bit matrix cores (the "x6" entry points; the name is older than the split).
-// Both operands are held as pairs of f16 planes of scaled values (f16_pair.h), x s = x0 + x1 to about
-// 2^-23 |x s|, and the product keeps three of the four plane products,
-//   a b s = a0 b0 + (a0 b1 + a1 b0) + e,   |e| = |a1 b1| <= 2^-22 |a0 b0|,
-// each exact in the fp32 accumulator of v_mfma_f32_32x32x16_f16.  That is half the products of a split
-// into three bf16 planes (six), with about the same representation error as one fp32 rounding per operand
-// and a third of the roundings into the accumulator.  f16 has five exponent bits, so the planes are scaled by
-// powers of two: A's by the largest magnitude of (row, 1024 columns of K), found where A is packed; B's by a
-// running scale per column that its wave finds as it goes.  A's scale changes along K, so each chunk's sum
-// is added, unscaled, to a second set of accumulators, which also shortens the chains of roundings.
+// fp32 product on the bf16 matrix cores ("x6").  Every fp32 operand x is split into three bf16
+// planes,
+//   x0 = rn(x), x1 = rn(x - x0), x2 = rn(x - x0 - x1)   (rn: round to nearest bf16)
+// with |x1| <= 2^-8 |x|, |x2| <= 2^-16 |x| and |x - x0 - x1 - x2| <= 2^-24 |x|, and the product keeps
+// the six plane products of order >= 2^-16 |a||b|:
+//   a b = a0 b0 + (a0 b1 + a1 b0) + (a0 b2 + a1 b1 + a2 b0) + e,   |e| <= ~2^-22.4 |a||b|
+// (a1 b2 + a2 b1 + a2 b2 and the residues below the third planes), the size of one or two fp32
+// roundings of the product; a product of two bf16 values is exact in the fp32 accumulator.
+// v_mfma_f32_32x32x16_bf16 has 16x the flop rate of v_mfma_f32_32x32x2_f32, so the six products
+// of a 32x32x16 step take 3/8 of the fp32 instruction time.
 //
 // Operands are packed into 128-row x 16-k tiles in MFMA fragment order: chunk c = (blk*2 + h)*32 + r
 // of a tile holds row blk*32 + r at k = 16 ks + 8 h + (0..7).  B (the large, reused operand) is
 // packed once as fp32 [N/128][K/16][2][256 chunks][4] (first and second four k of every chunk in two
-// 4 KB halves, so a fragment is two conflict-free 16-byte LDS reads); as f16 pairs it would take the same
-// bytes but need its column scales at hand.  A (small, re-formed per product) is packed as planes
-// [ceil(M/128)][K/16][2][256][8] and its reciprocal scales.  A work-group (128 x 128 tile, one K slice, four
-// waves of 128 x 32) reads each K slab as contiguous 8 KB (A, L2-resident) + 8 KB (B); every wave splits only
-// its own 32 columns of B and runs 12 MFMAs per slab.  Split s of tile t is block t * splits + s, so with
+// 4 KB halves, so a fragment is two conflict-free 16-byte LDS reads); A (small, re-formed per
+// product) is split and packed as bf16 planes [ceil(M/128)][K/16][3][256][8].  A work-group
+// (128 x 128 tile, one K slice, 2 x 2 waves of 64 x 64) reads each K slab as contiguous 12 KB (A,
+// L2-resident) + 8 KB (B) and runs 24 MFMAs per wave per slab.  gemm_x6_ring_kernel moves the slabs
+// with global_load_lds into a 4-stage LDS ring (three slabs in flight, no register staging), its
+// four waves take 128 x 32 each (1 x 4), and each wave splits its own B fragments; gemm_x6_kernel (K slices of an even slab count) stages through
+// registers and splits B once on its way to LDS.  Split s of tile t is block t * splits + s, so with
 // 8 or 16 splits every XCD (blocks are dispatched round-robin over 8) works on one or two K slices
 // and its L2 holds those slices of A.
-//
-// Bound at 128 rows: reading B.  128 x 14336 x 14336 (4 splits): 278 -> 206 us (4.0 TB/s of B; the
-// card copies at 4.7), 128 x 8192 x 8192 95 -> 74, 128 x 4096 x 4096 26.7 -> 23.4, against the six bf16 products of
-// the same tiling, with a relative error of 3.6e-7 against 9.9e-7 at 14336 (fp32 MFMA 7.6e-7).  At 4096 rows, bound
-// by the matrix cores: 4096 x 14336 x 14336 7.99 -> 5.56 ms.
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
 
 
 // B tiles: thread per chunk (8 floats).  trans_b: op(B)(k, n) = B[n*ldb + k] (32 contiguous bytes
@@ -506,201 +505,281 @@ __global__ void x6_pack_b_kernel(const float* __restrict__ B, int64_t ldb, int64
   }
 }
 
-// A pairs (of A diag(colscale) when colscale is given): work-group per (row, 1024 columns); rows >= M
-// are zero.
-__global__ __launch_bounds__(kThreads) void x6_pack_a_kernel(const float* __restrict__ A, int64_t lda, int64_t M,
-                                                             int64_t K, uint4* __restrict__ At,
-                                                             const float* __restrict__ colscale, int chunks,
-                                                             bool vec4) {
-  __shared__ float red[4];
-  const int64_t b = blockIdx.x / chunks;
-  const int64_t chunk = blockIdx.x - b * chunks;
-  const int64_t j0 = chunk * kPairChunk + 4 * (int64_t)threadIdx.x;
-  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (b < M && j0 < K) {
-    const float* src = A + b * lda + j0;
-    if (vec4) v = *reinterpret_cast<const float4*>(src);
-    else v = make_float4(src[0], src[1], src[2], src[3]);
-    if (colscale) {
-      v.x *= colscale[j0];
-      v.y *= colscale[j0 + 1];
-      v.z *= colscale[j0 + 2];
-      v.w *= colscale[j0 + 3];
+// A planes (of A diag(colscale) when colscale is given): thread per chunk; rows >= M are zero.
+__global__ void x6_pack_a_kernel(const float* __restrict__ A, int64_t lda, int64_t M, int64_t K, uint4* __restrict__ At,
+                                 const float* __restrict__ colscale) {
+  const int64_t KS = K / 16;
+  const int64_t nchunks = ((M + 127) / 128) * KS * 256;
+  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < nchunks; q += (int64_t)gridDim.x * blockDim.x) {
+    const int c = (int)(q & 255);
+    const int64_t tk = q >> 8;  // mt * KS + ks
+    const int64_t mt = tk / KS, ks = tk - mt * KS;
+    const int64_t m = mt * 128 + (c >> 6) * 32 + (c & 31), k0 = ks * 16 + ((c >> 5) & 1) * 8;
+    float v[8];
+    if (m < M) {
+      const float* src = A + m * lda + k0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = src[e];
+      if (colscale) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] *= colscale[k0 + e];
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = 0.f;
     }
+    uint4 h, mm, l;
+    split3(v[0], v[1], h.x, mm.x, l.x);
+    split3(v[2], v[3], h.y, mm.y, l.y);
+    split3(v[4], v[5], h.z, mm.z, l.z);
+    split3(v[6], v[7], h.w, mm.w, l.w);
+    uint4* d = At + tk * 768 + c;
+    d[0] = h;
+    d[256] = mm;
+    d[512] = l;
   }
-  pack_pair_chunk(At, M, K, b, chunk, v, red);
+}
+
+// C[split] (rows < M) = A[:, K slice] * op(B)[K slice, :] from the packed operands.  Every K slice
+// is an even number of 16-k slabs.
+__global__ __launch_bounds__(kThreads) void gemm_x6_kernel(int64_t M, int64_t N, int64_t K, const uint4* __restrict__ At,
+                                                           const float* __restrict__ Bt, float* __restrict__ C,
+                                                           int64_t ldc, int64_t split_stride, int64_t k_per_split,
+                                                           int splits) {
+  __shared__ uint4 As[2][3][256];
+  __shared__ uint4 Bs[2][3][256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wmb = (wave >> 1) * 2, wnb = (wave & 1) * 2;  // 2 x 2 waves of 64 x 64
+  const int64_t bid = blockIdx.x;
+  const int split = (int)(bid % splits);
+  const int64_t tile = bid / splits;
+  const int64_t ntn = N / 128;
+  const int64_t mt = tile / ntn, nt = tile - mt * ntn;
+  const int64_t KS = K / 16;
+  const int nslab = (int)(k_per_split / 16);
+  const int64_t ks0 = (int64_t)split * nslab;
+  // A slab: 768 chunks (3 planes), thread -> chunks tid + 256 j; B slab: 2 x 256 float4, thread ->
+  // both halves of chunk tid
+  const u32x4v* asrc = reinterpret_cast<const u32x4v*>(At) + (mt * KS + ks0) * 768 + tid;
+  const f32x4v* bsrc = reinterpret_cast<const f32x4v*>(Bt) + (nt * KS + ks0) * 512 + tid;
+
+  u32x4v qa0[3], qa1[3];
+  f32x4v qb0[2], qb1[2];
+  auto gload = [&](u32x4v (&qa)[3], f32x4v (&qb)[2], int64_t s) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) qa[j] = asrc[s * 768 + j * 256];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) qb[j] = bsrc[s * 512 + j * 256];
+  };
+  auto lstore = [&](const u32x4v (&qa)[3], const f32x4v (&qb)[2], int buf) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) As[buf][j][tid] = __builtin_bit_cast(uint4, qa[j]);
+    uint4 h, m, l;
+    split3(qb[0].x, qb[0].y, h.x, m.x, l.x);
+    split3(qb[0].z, qb[0].w, h.y, m.y, l.y);
+    split3(qb[1].x, qb[1].y, h.z, m.z, l.z);
+    split3(qb[1].z, qb[1].w, h.w, m.w, l.w);
+    Bs[buf][0][tid] = h;
+    Bs[buf][1][tid] = m;
+    Bs[buf][2][tid] = l;
+  };
+
+  floatx16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+  auto compute = [&](int buf) {
+    bf16x8 a[3][2], b[3][2];
+#pragma unroll
+    for (int pl = 0; pl < 3; ++pl) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) a[pl][i] = __builtin_bit_cast(bf16x8, As[buf][pl][(wmb + i) * 64 + lane]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) b[pl][j] = __builtin_bit_cast(bf16x8, Bs[buf][pl][(wnb + j) * 64 + lane]);
+    }
+    // smallest terms first; the (i, j) loop innermost keeps four independent accumulator chains
+    constexpr int pa[6] = {2, 1, 0, 1, 0, 0};
+    constexpr int pb[6] = {0, 1, 2, 0, 1, 0};
+#pragma unroll
+    for (int t = 0; t < 6; ++t)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[t]][i], b[pb[t]][j], acc[i][j], 0, 0, 0);
+  };
+
+  // same two-slabs-in-flight schedule as gemm_f32_full_kernel
+  gload(qa0, qb0, 0);
+  gload(qa1, qb1, 1);
+  lstore(qa0, qb0, 0);
+  __syncthreads();
+  for (int s = 0; s < nslab; s += 2) {
+    if (s + 2 < nslab) gload(qa0, qb0, s + 2);
+    compute(0);
+    lstore(qa1, qb1, 1);
+    __syncthreads();
+    if (s + 3 < nslab) gload(qa1, qb1, s + 3);
+    compute(1);
+    if (s + 2 < nslab) lstore(qa0, qb0, 0);
+    __syncthreads();
+  }
+
+  // lane l, accumulator v -> row 8*(v/4) + 4*(l/32) + v%4, column l%32 of the 32 x 32 block
+  const int col = lane & 31, rbase = (lane >> 5) * 4;
+  float* Cs = C + (int64_t)split * split_stride;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int64_t gn = nt * 128 + (wnb + j) * 32 + col;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int64_t gm = mt * 128 + (wmb + i) * 32 + (v >> 2) * 8 + rbase + (v & 3);
+        if (gm < M) Cs[gm * ldc + gn] = acc[i][j][v];
+      }
+    }
 }
 
 // s_waitcnt immediate that waits for vmcnt <= n only (gfx9 encoding: vmcnt bits 3:0 and 15:14).
 constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
-// C[split] (rows < M) = A[:, K slice] * op(B)[K slice, :] from the packed operands, the slabs moved by
-// global_load_lds into a ring of four LDS
+// Same product as gemm_x6_kernel with the slabs moved by global_load_lds into a ring of four LDS
 // stages (three slabs in flight, no register staging).  Each stage is its own __shared__ array and
 // the loops are unrolled by four, so every stage index is a constant: the compiler then tells the
 // stages apart and waits only where this code waits (s_waitcnt vmcnt(n) before each barrier: all
 // but the n most recent loads of this wave done, i.e. the slab about to be read).  The barrier is
 // s_barrier without a fence (the fence of __syncthreads would wait for every load in flight).
-// kRagged: K slices of any number of slabs; otherwise every slice is a positive multiple of four.
-// kStream: B is read with the non-temporal hint (it does not fit the caches anyway).
-template <bool kRagged, bool kStream>
-__global__ __launch_bounds__(kThreads, 2) void gemm_x6_kernel(int64_t M, int64_t N, int64_t K,
-                                                              const uint4* __restrict__ At,
-                                                              const float* __restrict__ Bt, float* __restrict__ C,
-                                                              int64_t ldc, int64_t split_stride,
-                                                              int64_t k_per_split, int splits) {
+// Every K slice is a positive multiple of four slabs.
+template <bool kColWaves>
+__global__ __launch_bounds__(kThreads) void gemm_x6_ring_kernel(int64_t M, int64_t N, int64_t K,
+                                                                const uint4* __restrict__ At,
+                                                                const float* __restrict__ Bt, float* __restrict__ C,
+                                                                int64_t ldc, int64_t split_stride,
+                                                                int64_t k_per_split, int splits) {
   constexpr int S = 4;
-  constexpr int STAGE = 512 + 512;  // 16-byte slots: A planes, then the two halves of B
-  constexpr int LOADS = 4;          // global_load_lds per wave per slab: 2 (A) + 2 (B)
-  constexpr int RT = 4;             // 32-row tiles of a wave (128 x 32)
-  constexpr int FAC = 16;           // chunks of A's scales kept in LDS
+  constexpr int STAGE = 768 + 512;  // 16-byte slots: A planes, then the two halves of B
+  constexpr int LOADS = 5;          // global_load_lds per wave per slab: 3 (A) + 2 (B)
   __shared__ uint4 st0[STAGE];
   __shared__ uint4 st1[STAGE];
   __shared__ uint4 st2[STAGE];
   __shared__ uint4 st3[STAGE];
-  __shared__ float fac[FAC][128];
   auto stage = [&](int slot) -> uint4* { return slot == 0 ? st0 : slot == 1 ? st1 : slot == 2 ? st2 : st3; };
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const unsigned utile = blockIdx.x / (unsigned)splits, ntn = (unsigned)(N / 128);  // 32-bit divisions: short
-  const int split = (int)(blockIdx.x - utile * (unsigned)splits);
-  const int64_t mt = utile / ntn, nt = utile % ntn;
+  // wave tiles: 2 x 2 waves of 64 x 64, or (kColWaves) 1 x 4 waves of 128 x 32: every wave splits
+  // only its own 32 columns of B (half the split work; the A planes, already split, are read by all
+  // four).  The launch uses the 1 x 4 form: the same products in the same order (bit-identical
+  // partials), 2.5-9 % less time at 128 x n x n for n = 4096, 8192 and 14336.
+  constexpr int RT = kColWaves ? 4 : 2, CT = kColWaves ? 1 : 2;
+  const int wmb = kColWaves ? 0 : (wave >> 1) * 2, wnb = kColWaves ? wave : (wave & 1) * 2;
+  const int64_t bid = blockIdx.x;
+  const int split = (int)(bid % splits);
+  const int64_t tile = bid / splits;
+  const int64_t ntn = N / 128;
+  const int64_t mt = tile / ntn, nt = tile - mt * ntn;
   const int64_t KS = K / 16;
   const int nslab = (int)(k_per_split / 16);
   const int64_t ks0 = (int64_t)split * nslab;
-  // wave w moves A slots w*128 + 64 q and B slots w*128 + 64 q (q < 2); lane l adds 16 l bytes
-  const uint4* asrc = At + (mt * KS + ks0) * 512 + wave * 128 + lane;
+  // wave w moves A slots w*192 + 64 q (q < 3) and B slots w*128 + 64 q (q < 2); lane l adds 16 l bytes
+  const uint4* asrc = At + (mt * KS + ks0) * 768 + wave * 192 + lane;
   const uint4* bsrc = reinterpret_cast<const uint4*>(Bt) + (nt * KS + ks0) * 512 + wave * 128 + lane;
   auto issue = [&](int s, int slot) {
     uint4* d = stage(slot);
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
-      __builtin_amdgcn_global_load_lds(asrc + (int64_t)s * 512 + q * 64, d + wave * 128 + q * 64, 16, 0, 0);
+    for (int q = 0; q < 3; ++q)
+      __builtin_amdgcn_global_load_lds(asrc + (int64_t)s * 768 + q * 64, d + wave * 192 + q * 64, 16, 0, 0);
 #pragma unroll
     for (int q = 0; q < 2; ++q)
-      __builtin_amdgcn_global_load_lds(bsrc + (int64_t)s * 512 + q * 64, d + 512 + wave * 128 + q * 64, 16, 0,
-                                       kStream ? 2 : 0);
+      __builtin_amdgcn_global_load_lds(bsrc + (int64_t)s * 512 + q * 64, d + 768 + wave * 128 + q * 64, 16, 0, 0);
   };
-  // slabs past the end of the slice are the last one again (never multiplied), so every step issues the
-  // same number of loads and waits for the same count
-  auto clamp_slab = [&](int t) { return t < nslab ? t : nslab - 1; };
-  // reciprocal scales of A's rows in the chunks of this slice: loaded before the first slabs, in LDS
-  // some barriers before they are read
-  const int64_t Mp = (M + 127) / 128 * 128;
-  const float* inv = reinterpret_cast<const float*>(At + Mp * K / 4) + mt * 128;
-  const int c0 = (int)(ks0 >> 6), nch = (int)((ks0 + nslab - 1) >> 6) - c0 + 1;  // kPairChunk = 64 slabs
-  float fq[FAC / 2];
-#pragma unroll
-  for (int q = 0; q < FAC / 2; ++q) {
-    const int c = 2 * q + (tid >> 7);
-    fq[q] = inv[(c0 + (c < nch ? c : nch - 1)) * Mp + (tid & 127)];
-  }
-#pragma unroll
-  for (int t = 0; t < S - 1; ++t) issue(clamp_slab(t), t);
-#pragma unroll
-  for (int q = 0; q < FAC / 2; ++q) fac[2 * q + (tid >> 7)][tid & 127] = fq[q];
-
-  floatx16 acc[RT], total[RT];
+  floatx16 acc[RT][CT];
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[i][v] = total[i][v] = 0.f;
-  // this lane's column of B (shared with lane ^ 32): scale, and the magnitude it holds up to.  The first
-  // nonzero slab sets the scale, with three bits to spare for larger values in later slabs.
-  float bs = 0x1p120f, blim = 60000.f * 0x1p-120f;
-  const int rbase = (lane >> 5) * 4;
-
-  // total += acc / (scales), for the chunk c of this slice
-  auto flush = [&](int c) {
-    const float binv = 1.f / bs;
+    for (int j = 0; j < CT; ++j)
 #pragma unroll
-    for (int i = 0; i < RT; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int r = i * 32 + q * 8 + rbase;
-        const float4 f = nch <= FAC ? *reinterpret_cast<const float4*>(&fac[c][r])
-                                    : *reinterpret_cast<const float4*>(inv + (int64_t)(c0 + c) * Mp + r);
-        const float fv[4] = {f.x, f.y, f.z, f.w};
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          total[i][4 * q + v] += acc[i][4 * q + v] * fv[v] * binv;
-          acc[i][4 * q + v] = 0.f;
-        }
-      }
-  };
-
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
   auto compute = [&](int slot) {
     const uint4* d = stage(slot);
-    f16x8 a[2][RT];
+    bf16x8 a[3][RT], b[3][CT];
 #pragma unroll
-    for (int pl = 0; pl < 2; ++pl)
+    for (int pl = 0; pl < 3; ++pl)
 #pragma unroll
-      for (int i = 0; i < RT; ++i) a[pl][i] = __builtin_bit_cast(f16x8, d[pl * 256 + i * 64 + lane]);
-    const float4 x = __builtin_bit_cast(float4, d[512 + wave * 64 + lane]);
-    const float4 y = __builtin_bit_cast(float4, d[512 + 256 + wave * 64 + lane]);
-    const float m = fmaxf(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))),
-                          fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w))));
-    if (__builtin_amdgcn_ballot_w64(m > blim)) {  // rare: a column outgrew its scale
-      const float mc = fmaxf(m, __shfl_xor(m, 32));
-      if (mc > blim && mc < INFINITY) {
-        const float ns = pair_scale(mc, 12);
-        const float f = ns / bs;
-        bs = ns;
-        blim = 60000.f / ns;
+      for (int i = 0; i < RT; ++i) a[pl][i] = __builtin_bit_cast(bf16x8, d[pl * 256 + (wmb + i) * 64 + lane]);
 #pragma unroll
-        for (int i = 0; i < RT; ++i)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) acc[i][v] *= f;
-      }
+    for (int j = 0; j < CT; ++j) {
+      const float4 x = __builtin_bit_cast(float4, d[768 + (wnb + j) * 64 + lane]);
+      const float4 y = __builtin_bit_cast(float4, d[768 + 256 + (wnb + j) * 64 + lane]);
+      uint4 h, m, l;
+      split3(x.x, x.y, h.x, m.x, l.x);
+      split3(x.z, x.w, h.y, m.y, l.y);
+      split3(y.x, y.y, h.z, m.z, l.z);
+      split3(y.z, y.w, h.w, m.w, l.w);
+      b[0][j] = __builtin_bit_cast(bf16x8, h);
+      b[1][j] = __builtin_bit_cast(bf16x8, m);
+      b[2][j] = __builtin_bit_cast(bf16x8, l);
     }
-    uint4 h, l;
-    split2(x.x, x.y, bs, h.x, l.x);
-    split2(x.z, x.w, bs, h.y, l.y);
-    split2(y.x, y.y, bs, h.z, l.z);
-    split2(y.z, y.w, bs, h.w, l.w);
-    const f16x8 b0 = __builtin_bit_cast(f16x8, h), b1 = __builtin_bit_cast(f16x8, l);
-    // smallest terms first; the row tiles innermost keep four independent accumulator chains
+    constexpr int pa[6] = {2, 1, 0, 1, 0, 0};
+    constexpr int pb[6] = {0, 1, 2, 0, 1, 0};
 #pragma unroll
-    for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1][i], b0, acc[i], 0, 0, 0);
+    for (int t = 0; t < 6; ++t)
 #pragma unroll
-    for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][i], b1, acc[i], 0, 0, 0);
+      for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0][i], b0, acc[i], 0, 0, 0);
+        for (int j = 0; j < CT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[t]][i], b[pb[t]][j], acc[i][j], 0, 0, 0);
   };
   auto sync = [&]() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  // slab t is the last of its chunk of A's scales, or of the slice
-  auto chunk_ends = [&](int t) { return t + 1 == nslab || ((ks0 + t) & 63) == 63; };
   // Slab t lives in stage t % 4.  Step t: wait for slab t (loads of slabs t+1, t+2 may stay in
   // flight), barrier (slab t visible; every wave is done with stage (t-1) % 4), issue slab t+3 into
-  // that stage, compute slab t.  One copy of the body, also for the last slabs: the code is fetched once
-  // per launch, and a short product spends a good part of its time on that.
-  for (int t0 = 0; t0 < nslab; t0 += S) {
+  // that stage, compute slab t.
+#pragma unroll
+  for (int t = 0; t < S - 1; ++t) issue(t, t);
+  int t0 = 0;
+  for (; t0 < nslab - S; t0 += S) {
 #pragma unroll
     for (int u = 0; u < S; ++u) {
-      const int t = t0 + u;
-      if (kRagged && t >= nslab) break;
       __builtin_amdgcn_s_waitcnt(vmcnt_imm(LOADS * (S - 2)));
       sync();
-      issue(clamp_slab(t + S - 1), (u + S - 1) % S);
+      issue(t0 + u + S - 1, (u + S - 1) % S);
       compute(u);
-      if ((kRagged || u == S - 1) && chunk_ends(t)) flush((int)((ks0 + t) >> 6) - c0);  // slices start at
-      // multiples of four slabs, so without kRagged chunks end with the last step
     }
   }
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // no load may land in LDS after the work-group ends
+  // last four slabs: slab nslab - 1 is issued in the first step, then the ring drains
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(LOADS * 2));
+  sync();
+  issue(t0 + S - 1, S - 1);
+  compute(0);
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(LOADS * 2));
+  sync();
+  compute(1);
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(LOADS * 1));
+  sync();
+  compute(2);
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  sync();
+  compute(3);
 
-  const int col = lane & 31;
+  const int col = lane & 31, rbase = (lane >> 5) * 4;
   float* Cs = C + (int64_t)split * split_stride;
-  const int64_t gn = nt * 128 + wave * 32 + col;
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int64_t gm = mt * 128 + i * 32 + (v >> 2) * 8 + rbase + (v & 3);
-      if (gm < M) Cs[gm * ldc + gn] = total[i][v];
+    for (int j = 0; j < CT; ++j) {
+      const int64_t gn = nt * 128 + (wnb + j) * 32 + col;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int64_t gm = mt * 128 + (wmb + i) * 32 + (v >> 2) * 8 + rbase + (v & 3);
+        if (gm < M) Cs[gm * ldc + gn] = acc[i][j][v];
+      }
     }
 }
 
@@ -809,11 +888,9 @@ hipError_t x6_pack_b(const float* B, int64_t ldb, bool trans_b, int64_t K, int64
 
 hipError_t x6_pack_a(const float* A, int64_t lda, int64_t M, int64_t K, void* At, hipStream_t stream,
                      const float* colscale) {
-  const int64_t chunks = (K + kPairChunk - 1) / kPairChunk, blocks = (M + 127) / 128 * 128 * chunks;
-  if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  const bool vec4 = (reinterpret_cast<uintptr_t>(A) & 15u) == 0 && lda % 4 == 0;
-  hipLaunchKernelGGL(x6_pack_a_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, A, lda, M, K,
-                     static_cast<uint4*>(At), colscale, (int)chunks, vec4);
+  const unsigned g = grid_for(((M + 127) / 128) * (K / 16) * 256);
+  hipLaunchKernelGGL(x6_pack_a_kernel, dim3(g), dim3(256), 0, stream, A, lda, M, K, static_cast<uint4*>(At),
+                     colscale);
   return hipGetLastError();
 }
 
@@ -823,14 +900,12 @@ hipError_t x6_gemm_partials(const void* At, const float* Bt, int64_t M, int64_t 
   if (!x6_shape_ok(N, K) || splits < 1 || K % splits != 0 || kps % 32 != 0) return hipErrorInvalidValue;
   const int64_t blocks = ((M + 127) / 128) * (N / 128) * splits;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  // An operator larger than the 256 MB last-level cache is gone before the next product reads it, and only
-  // pushes the other operands out: 128 x 14336 x 14336 takes 199 us with the hint and 210 without; 4096 x 4096
-  // (64 MB, which stays cached between products) 31.1 with and 28.2 without.
-  const bool ragged = (kps / 16) % 4 != 0, big = K * N * 4 >= ((int64_t)256 << 20);
-  const auto kernel = ragged ? (big ? gemm_x6_kernel<true, true> : gemm_x6_kernel<true, false>)
-                             : (big ? gemm_x6_kernel<false, true> : gemm_x6_kernel<false, false>);
-  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, M, N, K, static_cast<const uint4*>(At),
-                     Bt, C, ldc, split_stride, kps, splits);
+  if ((kps / 16) % 4 == 0)
+    hipLaunchKernelGGL(gemm_x6_ring_kernel<true>, dim3((unsigned)blocks), dim3(kThreads), 0, stream, M, N, K,
+                       static_cast<const uint4*>(At), Bt, C, ldc, split_stride, kps, splits);
+  else
+    hipLaunchKernelGGL(gemm_x6_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, M, N, K,
+                       static_cast<const uint4*>(At), Bt, C, ldc, split_stride, kps, splits);
   return hipGetLastError();
 }
 

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kEW) void uniform_denoise_kernel(
   if (MODE == kHardMap || MODE == kHardRoundMean) {
     if (planes) {  // uniform: the planes of the hard state for its x6 product
       __syncthreads();
-      chunk_planes(planes, gridDim.y, n, b, s_v, red);
+      chunk_planes(planes, n, b, s_v);
     }
   }
   if (MODE == kPosterior) {
@@ -183,7 +183,6 @@ __global__ __launch_bounds__(kEW) void epi2_denoise_kernel(
     const float* __restrict__ scale, const float* __restrict__ zero, int64_t G, int64_t gs, int maxq, float tau,
     uint8_t* __restrict__ q_out, float* __restrict__ x_out, uint4* __restrict__ planes) {
   static_assert(HMODE == kHardMap || HMODE == kHardRoundMean, "hard decision modes");
-  __shared__ float red[kEW / 64];
   __shared__ __attribute__((aligned(16))) float s_v[kChunk];
   const int64_t b = blockIdx.y;
   const float e2 = eta2[b], gb = g2[b], gn = g1new[b];
@@ -219,7 +218,7 @@ __global__ __launch_bounds__(kEW) void epi2_denoise_kernel(
   }
   if (planes) {
     __syncthreads();
-    chunk_planes(planes, gridDim.y, n, b, s_v, red);
+    chunk_planes(planes, n, b, s_v);
   }
 }
 
@@ -237,7 +236,7 @@ struct Workspace {
   float* prod_cur;   // xs Vs of the current / best hard state (kept when the caller asks for it)
   float* prod_best;
   float* P;   // split-K partials
-  void* Ap;   // packed f16 pairs of the left operand (x6 products)
+  void* Ap;   // packed bf16 planes of the left operand (x6 products)
   float* rowbuf;  // per-row arrays
   float* part;    // chunk partials (3 per row per chunk)
   uint8_t* q_cur;
@@ -323,7 +322,7 @@ VampStatus* host_status() {
 enum RankOperand : int { kOpV = 0, kOpVt = 1, kOpVs = 2 };
 
 // P = A @ op(B) as split-K partials into w.P (split_stride rows*n, w.splits of them).  With a packed
-// operator the product runs on the f16 matrix cores (A split into pairs first), else on the
+// operator the product runs on the bf16 matrix cores (A split into planes first), else on the
 // fp32 MFMA kernel.
 static hipError_t product(const Workspace& w, const float* A, const float* B, bool trans_b, RankOperand op,
                           int64_t rows, int64_t n, hipStream_t stream, bool a_planes_written = false) {
@@ -359,7 +358,7 @@ int uniform_vamp_solve(const UniformProblem& pr, const float* Vs, const MpqUnifo
     w.packed = pr.packed;
     w.splits = w.splits_x6;
   }
-  // x6 path: the kernels producing the left operands of the products write its f16 planes
+  // x6 path: the kernels producing the left operands of the products write its bf16 planes
   uint4* const planes = w.packed ? static_cast<uint4*>(w.Ap) : nullptr;
   const float* Yu = pr.Yu_in ? pr.Yu_in : w.Yu;
   VampStatus* hs = host_status();

@@ -8,7 +8,7 @@
 #include <cstring>
 
 #include "common.h"
-#include "f16_pair.h"
+#include "x6_split.h"
 
 namespace mpq {
 namespace {
@@ -56,17 +56,15 @@ __device__ __forceinline__ void publish_to(const VampStatus* st, StatusMailbox* 
   __hip_atomic_store(&box->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-static_assert(kChunk == kPairChunk && kEW == 256, "a work-group's columns are one scale group of the packed operand");
-
-// Pair planes of this work-group's column chunk of row b (of `rows`), staged in s_v (column
+// bf16 planes of this work-group's column chunk of row b, staged in s_v (column
 // blockIdx.x * kChunk + i at s_v[i]), at their place in the packed left operand At of the next x6
 // product (n % 16 == 0).  The producing kernels write them so the product needs no packing launch.
-// All threads call it; `red`: 4 floats of LDS.
-__device__ __forceinline__ void chunk_planes(uint4* __restrict__ At, int64_t rows, int64_t n, int64_t b,
-                                             const float* s_v, float* red) {
-  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-  if ((int64_t)blockIdx.x * kChunk + 4 * threadIdx.x < n) v = *reinterpret_cast<const float4*>(s_v + 4 * threadIdx.x);
-  pack_pair_chunk(At, rows, n, b, blockIdx.x, v, red);
+__device__ __forceinline__ void chunk_planes(uint4* __restrict__ At, int64_t n, int64_t b, const float* s_v) {
+  const int64_t j0 = (int64_t)blockIdx.x * kChunk + 4 * threadIdx.x;
+  if (j0 < n) {
+    const float4 v = *reinterpret_cast<const float4*>(s_v + 4 * threadIdx.x);
+    store_planes4(At, n, b, j0, v.x, v.y, v.z, v.w);
+  }
 }
 
 __global__ __launch_bounds__(64) void publish_status_kernel(const VampStatus* __restrict__ src,
@@ -235,7 +233,6 @@ __global__ __launch_bounds__(kEW) void msg_r2_kernel(int64_t n, const float* __r
                                                      const float* __restrict__ g2new, int has_prev,
                                                      float damping, const float* __restrict__ r2prev,
                                                      float* __restrict__ r2, uint4* __restrict__ planes) {
-  __shared__ float red[kEW / 64];
   __shared__ __attribute__((aligned(16))) float s_v[kChunk];
   const int64_t b = blockIdx.y;
   const float e1 = eta1[b], gw = g1w[b], gn = g2new[b];
@@ -253,7 +250,7 @@ __global__ __launch_bounds__(kEW) void msg_r2_kernel(int64_t n, const float* __r
   }
   if (planes) {  // uniform
     __syncthreads();
-    chunk_planes(planes, gridDim.y, n, b, s_v, red);
+    chunk_planes(planes, n, b, s_v);
   }
 }
 
@@ -291,7 +288,7 @@ __global__ __launch_bounds__(kEW) void lmmse_epi1_kernel(
   }
   if (planes) {  // uniform
     __syncthreads();
-    chunk_planes(planes, gridDim.y, n, b, s_v, red);
+    chunk_planes(planes, n, b, s_v);
   }
   const float t0 = block_sum(sinv, red);
   const float t1 = block_sum(sres, red);

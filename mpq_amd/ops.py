@@ -153,8 +153,8 @@ def gemm_x6_pack_b(B: torch.Tensor, *, trans_b: bool = False) -> torch.Tensor:
 
 
 def gemm_x6(A: torch.Tensor, B_packed: torch.Tensor, N: int, *, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """C = A @ op(B) with op(B) packed by :func:`gemm_x6_pack_b`: fp32 product on the f16 matrix
-    cores (a pair of scaled f16 planes per operand, three plane products)."""
+    """C = A @ op(B) with op(B) packed by :func:`gemm_x6_pack_b`: fp32 product on the bf16 matrix
+    cores (three bf16 planes per operand, six plane products)."""
     dev = _dev(A, B_packed)
     A = _f32c(A)
     M, K = A.shape
@@ -173,7 +173,7 @@ def gemm_x6(A: torch.Tensor, B_packed: torch.Tensor, N: int, *, out: Optional[to
 
 
 def gemm_x6_pack_a(A: torch.Tensor) -> torch.Tensor:
-    """A (M x K, K % 32 == 0) split into scaled f16 pairs and packed for :func:`gemm_x6_splitk` (uint8 buffer)."""
+    """A (M x K, K % 32 == 0) split into bf16 planes and packed for :func:`gemm_x6_splitk` (uint8 buffer)."""
     dev = _dev(A)
     A = _f32c(A)
     M, K = A.shape
@@ -391,7 +391,7 @@ def uniform_vamp_solve(W, x_init, scale, zero, group_size, maxq, V, S, Vs, cfg, 
     """One row block of the uniform VAMP loop.  Returns (q uint8, x|None, err, rtn_err, stats dict).
     ``Yu`` = W Vs and ``xr`` = x_init Vs may come from the caller (formed once for all row blocks);
     ``xprod_out`` (rows x n, contiguous fp32) then receives x_best Vs of the returned codes.
-    ``packed`` (from :func:`rankspace_pack`) runs the solver's products on the f16 matrix cores.
+    ``packed`` (from :func:`rankspace_pack`) runs the solver's products on the bf16 matrix cores.
     ``q_out`` (uint8 rows x n), ``err_out`` and ``rtn_err_out`` (float32 rows), contiguous, receive the
     results in place of new tensors."""
     dev = _dev(W, x_init, scale, zero, V, S, Vs, Yu, xr, xprod_out, packed)
@@ -514,7 +514,7 @@ def e8p12_vamp_solve(Wr, hat_init, V, S, Vs, cfg, *, prior_scale: Optional[torch
                      obs_init: float = 0.0, want_state: bool = False, ws: Optional[torch.Tensor] = None,
                      packed: Optional[torch.Tensor] = None):
     """One row block of the E8P12 VAMP loop (no polish).  ``packed`` (from :func:`rankspace_pack`)
-    runs the solver's products on the f16 matrix cores.
+    runs the solver's products on the bf16 matrix cores.
 
     Returns (idx int64 (rows, n/8), hat (rows, n), err (rows), r1|None, gamma1|None, stats dict)."""
     dev = _dev(Wr, hat_init, V, S, Vs, prior_scale, packed)

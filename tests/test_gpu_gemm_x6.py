@@ -120,44 +120,35 @@ def test_gemm_x6_splitk_partials_sum_to_the_product(gpu):
         assert float((P[s].cpu().double() - ref).abs().max()) <= 2e-6 * float(ref.abs().max())
 
 
-def _pair_bound(A, B):
-    """Error bound of one product from the f16 pairs.  Each operand is held to 2^-23 relative, or absolutely
-    to 2^-39 of the largest of its row's 1024 columns (A: that one is scaled to 2^14 .. 2^15, and the low
-    plane's last subnormal bit is 2^-24) and 2^-37 of its column's largest (B: scaled to at least 2^12); the
-    dropped low x low product is 2^-22 relative.  The fp32 roundings of the sums stay below what is
-    left of 2^-20 relative for the sizes tested."""
-    M, K = A.shape
-    amax = torch.zeros_like(A)
-    for c in range(0, K, 1024):
-        amax[:, c:c + 1024] = A[:, c:c + 1024].abs().amax(1, keepdim=True)
-    bmax = B.abs().amax(0, keepdim=True).expand_as(B)
-    return 2.0 ** -20 * (A.abs() @ B.abs()) + 2.0 ** -39 * (amax @ B.abs()) + 2.0 ** -37 * (A.abs() @ bmax)
+def _plane_bound(A, B):
+    """Entry-wise bound: each operand is held to 2^-24 relative whatever stands beside it, the dropped plane products
+    are below 2^-22.4, and the roundings of the sums stay below what is left of 2^-20 for the sizes tested."""
+    return 2.0 ** -20 * (A.abs() @ B.abs())
 
 
 @pytest.mark.parametrize("M,N,K,splits", [
     (3, 128, 32, 1), (128, 128, 1024, 1), (129, 256, 1056, 1), (128, 128, 2112, 3), (100, 128, 96, 1),
-    (128, 128, 17 * 1024, 1),    # more chunks of A's scales than a work-group keeps in LDS
-    (65, 128, 17 * 1024 + 32, 1),  # the same with a ragged slab count
+    (128, 128, 17 * 1024, 1), (65, 128, 17 * 1024 + 32, 1),
     (128, 256, 3584, 1), (64, 128, 4096, 8)])
-def test_pair_product_slices_and_chunks(gpu, M, N, K, splits):
-    """Slab counts that are not multiples of the ring's four stages, one and many 1024-column chunks."""
+def test_plane_product_slices(gpu, M, N, K, splits):
+    """Slab counts that are and are not multiples of the ring's four stages; splits of the caller's choice."""
     g = torch.Generator().manual_seed(M + N + K)
     A = torch.randn(M, K, generator=g).double().to(gpu)
     B = torch.randn(K, N, generator=g).double().to(gpu)
     Ap, Bp = ops.gemm_x6_pack_a(A.float()), ops.gemm_x6_pack_b(B.float())
     P, _ = ops.gemm_x6_splitk(Ap, Bp, M, N, K, splits=splits)
-    assert bool(((P.double().sum(0) - A @ B).abs() <= _pair_bound(A, B)).all())
+    assert bool(((P.double().sum(0) - A @ B).abs() <= _plane_bound(A, B)).all())
 
 
-def test_pair_product_scales_follow_the_data(gpu):
-    """Chunks of A and columns of B over 60 orders of magnitude: zero slabs first, columns that grow and
-    shrink along K, values far below their group's largest (subnormal planes), zero rows and columns."""
+def test_plane_product_keeps_small_entries(gpu):
+    """Rows of A and columns of B over 60 orders of magnitude: zero slabs first, columns that grow and
+    shrink along K, values far below their row's or column's largest, zero rows and columns."""
     M, N, K = 128, 256, 4096
     g = torch.Generator().manual_seed(77)
     A = torch.randn(M, K, generator=g).double()
     B = torch.randn(K, N, generator=g).double()
     A[:32] *= 1e-30
-    A[32:64, 1024:2048] *= 1e12   # chunk maxima 1, 1e12, 1, 1
+    A[32:64, 1024:2048] *= 1e12
     A[64:96, 2048:] *= 1e-20
     A[96] = 0.0
     k = torch.arange(K, dtype=torch.float64).view(-1, 1)
@@ -171,12 +162,12 @@ def test_pair_product_scales_follow_the_data(gpu):
     B[:, 200] = 0.0
     A, B = A.float().double().to(gpu), B.float().double().to(gpu)
     C = ops.gemm_x6(A.float(), ops.gemm_x6_pack_b(B.float()), N).double()
-    err, bound = (C - A @ B).abs(), _pair_bound(A, B)
+    err, bound = (C - A @ B).abs(), _plane_bound(A, B)
     assert bool((err <= bound).all()), float((err / bound).nan_to_num(0).max())
     assert float(C[96].abs().max()) == 0.0 and float(C[:, 200].abs().max()) == 0.0
 
 
-def test_pair_product_non_finite_stays_in_its_row_and_column(gpu):
+def test_plane_product_non_finite_stays_in_its_row_and_column(gpu):
     M, N, K = 40, 128, 2048
     g = torch.Generator().manual_seed(5)
     A, B = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g)
@@ -186,3 +177,30 @@ def test_pair_product_non_finite_stays_in_its_row_and_column(gpu):
     bad = torch.zeros(M, N, dtype=torch.bool)
     bad[3], bad[7], bad[:, 11] = True, True, True
     assert not bool(torch.isfinite(C[bad]).any()) and torch.equal(C[~bad], C0[~bad])
+
+
+@pytest.mark.parametrize("a,b", [(1e35, 1e-10), (1e-10, 1e35), (1e32, 1e-30), (-1e37, 1e-2)])
+def test_plane_product_reaches_the_range_limits(gpu, a, b):
+    """Operands near either end of fp32's range whose product is an ordinary number: no scaling may overflow or
+    vanish on the way."""
+    M, N, K = 40, 128, 1024
+    A, B = torch.full((M, K), a, device=gpu), torch.full((K, N), b, device=gpu)
+    ref = A.double() @ B.double()
+    Bp = ops.gemm_x6_pack_b(B)
+    P, _ = ops.gemm_x6_splitk(ops.gemm_x6_pack_a(A), Bp, M, N, K)
+    for C in (ops.gemm_x6(A, Bp, N).double(), P.double().sum(0)):
+        assert float(((C - ref) / ref).abs().max()) < 2.0 ** -18
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (1, 128, 128), (100, 384, 384), (128, 1024, 1024), (256, 1152, 1152),
+                                   (128, 2048, 2048), (256, 2048, 2048)])
+def test_gemm_x6_small_products(gpu, M, N, K):
+    """Entry-wise error relative to sum_k |a_k b_k| of products with few work-groups: one rounding per MFMA of a
+    slice (6 per 16 k), one per partial summed and four for the split and the dropped plane products."""
+    g = torch.Generator().manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g) * torch.exp(2.0 * torch.randn(1, K, generator=g))
+    B = torch.randn(K, N, generator=g)
+    splits = ops._lib.load().mpq_gemm_x6_split_count(M, N, K)
+    C = ops.gemm_x6(A.to(gpu), ops.gemm_x6_pack_b(B.to(gpu)), N).cpu().double()
+    err = (C - A.double() @ B.double()).abs() / (A.double().abs() @ B.double().abs())
+    assert float(err.max()) <= (6 * K / (16 * splits) + splits + 4) * 2.0**-24

@@ -49,8 +49,8 @@ def stops(n, seed, device):
     return {"entered": st["vamp_iters_entered"], "best": st["vamp_iters"]}
 
 
-# two-stage decomposition, fp32 products
-@pytest.mark.parametrize("n,seed", [(2048, 73), (2048, 79), (1536, 10), (2048, 43), (2048, 75)])
+# two-stage decomposition and fp32 products; at 4096 the packed products
+@pytest.mark.parametrize("n,seed", [(2048, 73), (2048, 79), (1536, 10), (2048, 43), (2048, 75), (4096, 4), (4096, 17)])
 def test_row_blocks_stop_where_they_did(gpu, n, seed):
     with open(GOLDEN) as f:
         want = json.load(f)[f"{n} {seed}"]
