@@ -383,7 +383,8 @@ int mpq_uniform_rtn(const float* W, int64_t rows, int64_t n, int64_t ldw, const 
  *     total row count for w_mean); workspace >= rows * n/group_size floats.
  *   mpq_awq_search: W rows x n, H n x n, x_mean n (mean |x|), w_mean n; outputs best_scales (n,
  *     device), losses_out (20, device, optional), best_error / best_ratio (host pointers,
- *     optional).  Synchronises `stream` once.  n % group_size == 0.
+ *     optional).  Synchronises `stream` once.  n % group_size == 0.  The workspace needs no more than the
+ *     alignment of a float.
  */
 int64_t mpq_awq_workspace_size(int64_t rows, int64_t n);
 int mpq_awq_w_mean(const float* W, int64_t rows, int64_t n, int64_t group_size, float* w_sum,

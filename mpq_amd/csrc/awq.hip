@@ -196,7 +196,8 @@ AwqPlan awq_plan(int64_t rows, int64_t n) {
   p.splits = p.x6 ? x6_choose_splits(rows, n, n) : choose_splits(rows, n, n, (int64_t)1 << 62, &p.bn);
   p.hp_bytes = p.x6 ? a64(n * n) * 4 : 0;
   p.ap_bytes = p.x6 ? (x6_packed_a_bytes(rows, n) + 255) / 256 * 256 : 0;
-  p.bytes = (a64(rows * n) * (1 + p.splits) + a64(rows) + 64 + a64(kRatios * n)) * 4 + p.hp_bytes + p.ap_bytes;
+  // 256 bytes to begin on a 256-byte boundary of any workspace: the packed operands move in 16-byte pieces
+  p.bytes = 256 + (a64(rows * n) * (1 + p.splits) + a64(rows) + 64 + a64(kRatios * n)) * 4 + p.hp_bytes + p.ap_bytes;
   return p;
 }
 
@@ -238,7 +239,7 @@ extern "C" int mpq_awq_search(const float* W, int64_t rows, int64_t n, const flo
   MPQ_CHECK_ARG(workspace_bytes >= mpq_awq_workspace_size(rows, n), "mpq_awq_search: workspace too small");
   MPQ_CHECK_ARG(rows <= 65535 * 128LL, "mpq_awq_search: too many rows");
   const AwqPlan pl = awq_plan(rows, n);
-  char* p = static_cast<char*>(workspace);
+  char* p = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(workspace) + 255) & ~(uintptr_t)255);
   float* D = (float*)p; p += a64(rows * n) * 4;
   float* P = (float*)p; p += a64(rows * n) * pl.splits * 4;
   float* rowq = (float*)p; p += a64(rows) * 4;

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from mpq_amd import awq
+from mpq_amd import awq, ops
 from oracle import awq as oa
 from tests.uniform_cases import make_layer
 
@@ -49,3 +49,27 @@ def test_search_on_packed_products_matches_fp64(gpu, rows, n):
     s, e, r, losses = awq.search_best_scale_linear(W.to(gpu), H.to(gpu), x_mean.to(gpu), bits=4, group_size=128)
     assert torch.allclose(losses.cpu(), torch.tensor(l_ref), rtol=2e-4)
     assert abs(r - r_ref) < 1e-6 and abs(e - e_ref) <= 2e-4 * e_ref and torch.allclose(s.cpu(), s_ref, rtol=1e-5)
+
+
+@pytest.mark.parametrize("n,group", [(1024, 128), (384, 64)])
+def test_search_takes_a_workspace_of_any_float_alignment(gpu, n, group):
+    """The packed operands want 16-byte pieces; a workspace that begins 4 bytes off gives the same losses."""
+    rows = 1100
+    g = torch.Generator().manual_seed(n)
+    W = (0.02 * torch.randn(rows, n, generator=g)).to(gpu)
+    X = torch.randn(2 * n, n, generator=g).to(gpu)
+    H, x_mean = (X.T @ X / (2 * n)).contiguous(), X.abs().mean(0)
+    w_mean = awq.compute_w_mean([W], group)
+    lib = ops._lib.load()
+    need = int(lib.mpq_awq_workspace_size(rows, n))
+
+    def losses(offset):
+        ws = torch.empty(need + 4096, dtype=torch.uint8, device=gpu).fill_(0xFF)
+        scales, out = torch.empty(n, device=gpu), torch.empty(20, device=gpu)
+        ops._lib.call("mpq_awq_search", ops._lib.ptr(W), rows, n, ops._lib.ptr(H), ops._lib.ptr(x_mean),
+                      ops._lib.ptr(w_mean), group, 4, 0, ops._lib.ptr(scales), ops._lib.ptr(out), 0, 0,
+                      ops._lib.ptr(ws[256 + offset:]), need, ops._lib.stream_handle(gpu))
+        assert bool((ws[:256 + offset] == 0xFF).all()) and bool((ws[256 + offset + need:] == 0xFF).all())
+        return out
+
+    assert torch.equal(losses(0), losses(4)) and torch.equal(losses(0), losses(252))
