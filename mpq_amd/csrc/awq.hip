@@ -180,9 +180,11 @@ namespace mpq {
 namespace {
 
 // The search's workspace.  The 20 products D H run as x6 products on H packed once (bf16 matrix cores) where
-// the shape has them; else, and for problems so small that the launches are what counts, on the fp32 kernel.
-// 4096 x 4096, the whole search: 23.8 ms with fp32 products, 14.9 with x6; below n = 1024 the extra
-// launches cost more than the product gains (4096 x 512: 1.27 ms with x6, 1.19 without; 2048 x 640: 1.15 / 1.12).
+// the shape has them and the products are large: packing H and the deltas, and the x6 grid's fewer K slices, cost
+// a small one more than the products gain.  The whole search with fp32 products / with x6, ms:
+//   64 x 2048 0.82 / 0.90, 256 x 1024 0.64 / 0.84, 4096 x 512 1.19 / 1.27, 2048 x 640 1.12 / 1.15 (fp32 taken);
+//   256 x 2048 0.93 / 0.96, 64 x 4096 1.65 / 1.07, 1000 x 1152 1.40 / 1.09, 2048 x 1024 1.50 / 1.29,
+//   2048 x 2048 3.82 / 2.71, 4096 x 4096 23.8 / 14.9 (x6 taken).
 struct AwqPlan {
   bool x6;
   int splits, bn;
@@ -192,7 +194,7 @@ struct AwqPlan {
 AwqPlan awq_plan(int64_t rows, int64_t n) {
   AwqPlan p{};
   p.bn = 128;
-  p.x6 = x6_shape_ok(n, n) && n >= 1024;
+  p.x6 = x6_shape_ok(n, n) && n >= 1024 && rows * n >= ((int64_t)1 << 30) / n;
   p.splits = p.x6 ? x6_choose_splits(rows, n, n) : choose_splits(rows, n, n, (int64_t)1 << 62, &p.bn);
   p.hp_bytes = p.x6 ? a64(n * n) * 4 : 0;
   p.ap_bytes = p.x6 ? (x6_packed_a_bytes(rows, n) + 255) / 256 * 256 : 0;

@@ -34,9 +34,10 @@ def test_search_matches_oracle(gpu, bits, sym):
     assert torch.allclose(s.cpu(), s_ref, rtol=1e-5)
 
 
-@pytest.mark.parametrize("rows,n", [(33, 1024), (130, 1152)])
+@pytest.mark.parametrize("rows,n", [(33, 1024), (130, 1152), (1025, 1024), (1023, 1024), (65, 4096)])
 def test_search_on_packed_products_matches_fp64(gpu, rows, n):
-    """From n = 1024 the products D H run as x6 products on H packed once; rows that are no whole tiles.  The
+    """From n = 1024 and rows n^2 = 2^30 the products D H run as x6 products on H packed once, below on the fp32
+    kernel; rows that are no whole tiles, both sides of the rule.  The
     losses against fp64 on the same scales and deltas' formula: a weight that rounds the other way moves a
     loss by less than 1e-4 at these sizes (the fp32 path's own bar is 2e-4)."""
     g = torch.Generator().manual_seed(rows)
