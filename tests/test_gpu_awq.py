@@ -17,6 +17,14 @@ def test_w_mean(gpu):
     assert torch.allclose(got, ref, rtol=2e-6, atol=1e-7)
 
 
+@pytest.mark.parametrize("rows,n,group", [(37, 960, 1), (37, 960, 2), (5, 960, 3), (37, 960, 5), (130, 960, 16),
+                                          (7, 960, 60), (3, 960, 64), (37, 960, 96), (1, 960, 960)])
+def test_w_mean_group_sizes(gpu, rows, n, group):
+    """One to 64 lanes per group; groups that fill no power of two, rows whose groups fill no wave."""
+    W = torch.randn(rows, n, generator=torch.Generator().manual_seed(group)) * 0.02
+    assert torch.allclose(awq.compute_w_mean([W.to(gpu)], group).cpu(), oa.compute_w_mean([W], group), rtol=2e-6, atol=1e-7)
+
+
 @pytest.mark.parametrize("bits,sym", [(4, False), (3, False), (4, True)])
 def test_search_matches_oracle(gpu, bits, sym):
     W, H = make_layer(96, 256, tokens=1024, seed_key=f"awq:{bits}:{sym}")
