@@ -249,6 +249,32 @@ def test_vamp_block_with_caller_products(gpu):
     assert _rel(a[1].cpu(), b[1].cpu()) < 1e-4 and _rel(a[2].cpu(), b[2].cpu()) < 1e-4
 
 
+@pytest.mark.parametrize("rows", [8, 104, 129, 200])
+def test_vamp_block_packed_ragged_rows(gpu, rows):
+    """Packed products of rows that are no whole 128-row tiles, workspace and outputs full of NaN before: codes
+    against the oracle, err and x_best Vs against fp64 of the returned codes."""
+    n = 512
+    W, Hw, V, S, Vs, sg, zg, sf, zf, xr, maxq = _setup_block(rows, n, 4, 128, f"packed:{rows}", rotate=True)
+    cfg = dict(RECIPE, polish_sweeps=0)
+    q_ref, _, e_ref, _, tr = ou.solve_uniform_rankspace_vamp(W, xr, sf, zf, maxq, V, V.T, S, Vs, cfg)
+    vcfg = UniformVampConfig(**{k: v for k, v in RECIPE.items()})
+    Vg, Vsg = V.to(gpu), Vs.to(gpu)
+    need = int(ops._lib.load().mpq_uniform_vamp_workspace_size(rows, n))
+    ws = torch.full((need + 4096,), 0xFF, dtype=torch.uint8, device=gpu)  # 0xFFFFFFFF: a NaN
+    nan = [torch.full(s, float("nan"), device=gpu) for s in ((rows, n), (rows,), (rows,))]
+    q, x, e, rtn, st = ops.uniform_vamp_solve(W.to(gpu), xr.to(gpu), sg.to(gpu), zg.to(gpu), 128, maxq, Vg, S.to(gpu),
+                                              Vsg, vcfg, want_x=True, packed=ops.rankspace_pack(Vg, Vsg),
+                                              ws=ws[:need], xprod_out=nan[0], err_out=nan[1], rtn_err_out=nan[2])
+    assert bool((ws[need:] == 0xFF).all())
+    assert float((q.cpu().long() == q_ref.long()).float().mean()) >= 0.999
+    assert st["best_iter"] == tr["best_iter"] and st["stop_iter"] == tr["stop_iter"]
+    Wd, xd, Vd = W.double(), x.cpu().double(), Vs.double()
+    assert torch.allclose(e.cpu().double(), ((Wd - xd) @ Vd).square().sum(1), rtol=1e-4)
+    assert torch.allclose(rtn.cpu().double(), ((Wd - xr.double()) @ Vd).square().sum(1), rtol=1e-4)
+    xp = xd @ Vd
+    assert float((nan[0].cpu().double() - xp).abs().max()) <= 2e-6 * float((xd.abs() @ Vd.abs()).max())
+
+
 def test_cd_polish_matches_oracle(gpu):
     W, Hw, V, S, Vs, sg, zg, sf, zf, xr, maxq = _setup_block(256, 512, 4, 128, "cd")
     q0 = torch.clamp(torch.round(W / sf) + zf, 0, maxq).to(torch.uint8)
@@ -352,7 +378,8 @@ def test_postprocess_gptq_polish_matches_oracle(gpu, layout):
     assert torch.equal(got, sf * (qf.cpu().float() - zf))
 
 
-def test_vamp_early_stop_then_call_on_another_stream(gpu):
+@pytest.mark.parametrize("packed", [False, True])
+def test_vamp_early_stop_then_call_on_another_stream(gpu, packed):
     """Status mailbox (two slots, one per pending publish): a block that stops at the best iterate
     leaves the look-ahead pass's status publish queued; the driver waits for it before returning, so
     a second call from the same thread on another stream, started right away, reads only its own
@@ -361,11 +388,12 @@ def test_vamp_early_stop_then_call_on_another_stream(gpu):
     for key in ("mb0", "mb3"):  # oracle: best-iterate stops at 7 and 9 of 16 iterations
         W, Hw, V, S, Vs, sg, zg, sf, zf, xr, maxq = _setup_block(128, 512, 4, 128, key, rotate=True)
         cases.append([t.to(gpu) for t in (W, xr, sg, zg)] + [maxq] + [t.to(gpu) for t in (V, S, Vs)])
+        cases[-1].append(ops.rankspace_pack(*cases[-1][5::2]) if packed else None)
     vcfg = UniformVampConfig(**{k: v for k, v in RECIPE.items()})
 
     def solve(c):
-        W, xr, sg, zg, maxq, V, S, Vs = c
-        return ops.uniform_vamp_solve(W, xr, sg, zg, 128, maxq, V, S, Vs, vcfg)
+        W, xr, sg, zg, maxq, V, S, Vs, pk = c
+        return ops.uniform_vamp_solve(W, xr, sg, zg, 128, maxq, V, S, Vs, vcfg, packed=pk)
 
     alone = [solve(c) for c in cases]
     torch.cuda.synchronize()
@@ -380,3 +408,14 @@ def test_vamp_early_stop_then_call_on_another_stream(gpu):
         assert torch.equal(got[0], ref[0])
         assert torch.equal(got[2], ref[2])
         assert got[4]["stop_iter"] == ref[4]["stop_iter"] and got[4]["best_iter"] == ref[4]["best_iter"]
+
+
+@pytest.mark.parametrize("M,N,K", [(104, 1000, 1000), (128, 256, 256), (1, 64, 64), (24, 104, 104), (129, 72, 2081),
+                                   (128, 512, 544), (128, 512, 512)])
+def test_gemm_small_products_split(gpu, M, N, K):
+    """The partials of the library's split count, last slices that are short among them, sum to the product."""
+    g = torch.Generator().manual_seed(M + N + K)
+    A, B = torch.randn(M, K, generator=g), torch.randn(K, N, generator=g)
+    for trans in (False, True):
+        P, _ = ops.gemm_splitk(A.to(gpu), (B.T.contiguous() if trans else B).to(gpu), trans_b=trans)
+        assert _rel(P.sum(0).cpu(), A.double() @ B.double()) < 2e-6
