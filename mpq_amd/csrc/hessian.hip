@@ -48,8 +48,13 @@ __global__ __launch_bounds__(kThreads, 2) void syrk_kernel(const void* __restric
   constexpr int KS = R * 128 / NQ;              // tokens per slab: 32 (16: fp32, TS = 128)
   constexpr int NB = TS / 64;                   // 32 x 32 blocks per wave and dimension
   constexpr int D = !kBf16 && TS == 128 ? 2 : 4;  // slabs of loads in flight (even)
-  __shared__ uint4 As[2][NP][KS / 8][TS];
-  __shared__ uint4 Bs[2][NP][KS / 8][TS];
+  union Lds {
+    uint4 op[2][2][NP][KS / 8][TS];
+    float out[TS / NB][TS];
+  };
+  __shared__ Lds lds;
+  auto& As = lds.op[0];
+  auto& Bs = lds.op[1];
 
   // upper-triangular tile index -> (ti, tj), ti <= tj: tj (tj + 1) / 2 tiles precede column tj
   const int t = (int)blockIdx.x;
@@ -216,23 +221,51 @@ __global__ __launch_bounds__(kThreads, 2) void syrk_kernel(const void* __restric
     }
   }
 
-  // elements on or above the diagonal are written to (m, n) and (n, m)
+  // Elements on or above the diagonal are written to (m, n) and (n, m), by way of LDS so that both are
+  // written along rows of H: straight from the accumulators they went out 16 bytes and, for (n, m), four rows
+  // apart (16 tokens, both with 128 x 128 tiles: 4096 bf16 88 -> 57 us, 8192 fp32 248 -> 161).  Chunk i holds the
+  // tile's rows NB lr + i; entry (lr, cn) is kept at column (cn + lr) % TS, so reads along either index spread over
+  // the banks.
+  constexpr int kBatch = 8;
 #pragma unroll
-  for (int i = 0; i < NB; ++i)
+  for (int i = 0; i < NB; ++i) {
+    if (i) __syncthreads();
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      const int64_t gn = n0 + col_of(sn + 32 * j);
+      const int cn = col_of(sn + 32 * j);
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int64_t gm = m0 + col_of((wave >> 1) * (TS / 2) + 32 * i + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3));
-        if (gn < gm) continue;
-        float* dst = H + gm * ldh + gn;
-        const float sum = acc[i][j][v];
-        const float val = beta == 0.f ? alpha * sum : alpha * sum + beta * *dst;
-        *dst = val;
-        if (gn != gm) H[gn * ldh + gm] = val;
+        const int lr = col_of((wave >> 1) * (TS / 2) + 32 * i + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3)) / NB;
+        lds.out[lr][(cn + lr) % TS] = alpha * acc[i][j][v];
       }
     }
+    __syncthreads();
+    for (int q0 = tid; q0 < TS / NB * TS; q0 += kBatch * kThreads) {
+      float old[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const int q = q0 + u * kThreads, lr = q / TS, cn = q % TS;
+        const int64_t gm = m0 + NB * lr + i, gn = n0 + cn;
+        old[u] = beta != 0.f && gn >= gm ? H[gm * ldh + gn] : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const int q = q0 + u * kThreads, lr = q / TS, cn = q % TS;
+        const int64_t gm = m0 + NB * lr + i, gn = n0 + cn;
+        if (gn < gm) continue;
+        float val = lds.out[lr][(cn + lr) % TS];
+        if (beta != 0.f) lds.out[lr][(cn + lr) % TS] = val = val + beta * old[u];
+        H[gm * ldh + gn] = val;
+      }
+    }
+    __syncthreads();
+#pragma unroll 8
+    for (int q = tid; q < TS / NB * TS; q += kThreads) {
+      const int cn = q / (TS / NB), lr = q % (TS / NB);
+      const int64_t gm = m0 + NB * lr + i, gn = n0 + cn;
+      if (gn > gm) H[gn * ldh + gm] = lds.out[lr][(cn + lr) % TS];
+    }
+  }
 }
 
 // colsum[j] += sum_t X[t][j], in a fixed order: a work-group owns 16 columns, thread (g, j) adds the
@@ -270,8 +303,12 @@ void launch(const void* X, int64_t T, int64_t n, int64_t ldx, float alpha, float
   // there 64 x 64 tiles (four times as many).  8192 tokens, 128 / 64 tiles, us: n = 1024 bf16 143 / 96,
   // fp32 460 / 195; 2304 (171 tiles) 152 / 132, 462 / 366; 2816 (253 tiles) 160 / 167, 478 / 521;
   // 4096 271 / 369, 1092 / 1058; 8192 935 / 1337, 3365 / 4233.
+  // Up to 256 tokens the time is that of reading and writing H, and smaller tiles spread it over more
+  // work-groups: 32 tokens, 128 / 64 tiles, us: 2560 bf16 43 / 30, fp32 43 / 39; 4096 55 / 42, 71 / 57; 8192
+  // 133 / 100, 158 / 153; 256 tokens: 2560 47 / 34, 56 / 51; 3584 53 / 45, 66 / 67; 8192 166 / 130, 242 / 226.  At
+  // 512 tokens 3584 59 / 52, 86 / 92; 8192 184 / 161, 331 / 352.
   const int64_t nt = n / 128, tiles = nt * (nt + 1) / 2;
-  if (tiles >= 200) {
+  if (tiles >= 200 && T > 256) {
     hipLaunchKernelGGL((syrk_kernel<kBf16, 128>), dim3((unsigned)tiles), dim3(kThreads), 0, stream, X, T, n, ldx,
                        alpha, beta, H, ldh);
   } else {

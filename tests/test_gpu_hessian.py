@@ -79,10 +79,11 @@ def test_rejects_bad_width(gpu):
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("T,n", [(1, 128), (31, 128), (33, 384), (127, 640), (129, 2432), (100, 2560)])
+@pytest.mark.parametrize("T,n", [(1, 128), (31, 128), (33, 384), (127, 640), (129, 2432), (100, 2560),
+                                 (256, 2560), (257, 2560), (271, 2560), (300, 2432)])
 def test_syrk_slab_and_tile_edges(gpu, T, n, bf16):
-    """Partial token slabs, the 64 x 64 tiles (below 200 tiles of 128 x 128: n <= 2432) and the 128 x 128
-    tiles, and the column sums.  Each entry sums T products exact to 2^-22 relative in fp32: its error is
+    """Partial token slabs, the 64 x 64 tiles (up to 256 tokens, or below 200 tiles of 128 x 128: n <= 2432) and
+    the 128 x 128 tiles, and the column sums.  Each entry sums T products exact to 2^-22 relative in fp32: its error is
     at most (2^-22 + (T + 2) 2^-24) sum |x_i x_j|."""
     g = torch.Generator().manual_seed(7 * T + n)
     X = torch.randn(T, n, generator=g) * torch.exp(torch.randn(n, generator=g))
@@ -97,11 +98,11 @@ def test_syrk_slab_and_tile_edges(gpu, T, n, bf16):
     assert bool(((cs.double() - 1 - Xd.sum(0)).abs() <= (T + 2) * 2.0 ** -24 * (1 + Xd.abs().sum(0))).all())
 
 
-@pytest.mark.parametrize("n", [256, 2560])
-def test_syrk_non_finite_activations(gpu, n):
+@pytest.mark.parametrize("T,n", [(40, 256), (40, 2560), (259, 2560)])
+def test_syrk_non_finite_activations(gpu, T, n):
     """Infinities, NaN and values that round to an infinity in bf16 act as in fp32 products."""
     g = torch.Generator().manual_seed(n)
-    X = torch.randn(40, n, generator=g)
+    X = torch.randn(T, n, generator=g)
     X[5, 7], X[9, 100], X[3, 50] = float("inf"), float("nan"), 3.4e38
     X[3, 7] = 0.5  # 3.4e38 X[3, 7] must not overflow before the infinity of column 7 is added (fp32 would give NaN)
     H = torch.zeros(n, n, device=gpu)
@@ -137,3 +138,23 @@ def test_syrk_non_finite_activations_cost_one_more_product(gpu):
     one[7, 5] = float("inf")
     assert best_ms(one) < 20 * finite
     assert best_ms(torch.full_like(X, float("inf"))) < 20 * finite
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("T,n", [(3, 2560), (300, 256), (300, 2560)])
+def test_syrk_adds_to_the_upper_triangle(gpu, T, n, bf16):
+    """H = beta H + alpha X^T X of both tile sizes: the entries on and above the diagonal count, the others are
+    written as their mirror image.  With H = 0, beta = 0 gives X^T X exactly as beta = 1 does."""
+    g = torch.Generator().manual_seed(T + n)
+    X = torch.randn(T, n, generator=g).to(torch.bfloat16 if bf16 else torch.float32).to(gpu)
+    H0 = torch.randn(n, n, generator=g).to(gpu)
+    H = hessian.accumulate(H0.clone(), X, alpha=0.75, beta=0.5)
+    upper = torch.triu(H0.double())
+    sym = upper + torch.triu(H0.double(), 1).T
+    Xd = X.double()
+    bound = 2.0 ** -23 * sym.abs() + (2.0 ** -22 + (T + 4) * 2.0 ** -24) * (Xd.abs().T @ Xd.abs())
+    assert bool(((H.double() - 0.5 * sym - 0.75 * Xd.T @ Xd).abs() <= bound).all())
+    assert torch.equal(H, H.T)
+    P1 = hessian.accumulate(torch.zeros_like(H0), X)
+    P0 = hessian.accumulate(torch.full_like(H0, float("nan")), X, beta=0.0)
+    assert torch.equal(P0, P1)
