@@ -187,10 +187,11 @@ def test_eigen_cache_exact_match_only(gpu):
 
 
 @pytest.mark.parametrize("n,dtype", [(1025, torch.float32), (1090, torch.float64), (2048, torch.float64),
-                                     (2115, torch.float64)])
+                                     (2115, torch.float64), (4170, torch.float64), (8260, torch.float32)])
 def test_one_stage_batch_sizes(gpu, n, dtype):
     """The finishing kernel's load batches change at 16, 32, 64 and 128 strips of 64 rows left: solves that
-    cross them, against the matrix itself (backward error and orthogonality n u, u the unit roundoff)."""
+    cross the first (n = 1025, 1090), the second (2115), the third (4170) and the last (8260), against the matrix
+    itself (backward error and orthogonality n u, u the unit roundoff)."""
     g = torch.Generator().manual_seed(n)
     A = torch.randn(n, n, generator=g, dtype=torch.float64)
     H = ((A + A.T) / 2).to(dtype).to(gpu)
