@@ -36,8 +36,8 @@ constexpr int kThreads = 256;
 //
 // Bound: bf16, the LDS fragment reads (1 KB per MFMA and wave with 64 x 64 wave tiles: the LDS rate);
 // fp32, the matrix cores (six products per fragment pair).  4096 columns x 16384 tokens
-// bf16: 4660 -> 575 us (478 TFLOP/s of n^2 T); 14336 x 8192 bf16: 18.7 -> 2.7 ms (616 TFLOP/s); 2048 x 3001
-// fp32: 221 -> 135 us, both against one fp32 MFMA kernel for either type.
+// bf16: 4780 -> 523 us (525 TFLOP/s of n^2 T); 14336 x 8192 bf16: 18.9 -> 2.57 ms (656 TFLOP/s); 2048 x 3001
+// fp32: 228 -> 140 us, all against one fp32 MFMA kernel for either type (repeated calls on one input).
 template <bool kBf16, int TS>
 __global__ __launch_bounds__(kThreads, 2) void syrk_kernel(const void* __restrict__ X, int64_t T, int64_t n,
                                                         int64_t ldx, float alpha, float beta,
@@ -300,9 +300,9 @@ template <bool kBf16>
 void launch(const void* X, int64_t T, int64_t n, int64_t ldx, float alpha, float beta, float* H, int64_t ldh,
             float* colsum, hipStream_t stream) {
   // 128 x 128 tiles read half as much LDS per product, but well below one tile per CU the chip idles:
-  // there 64 x 64 tiles (four times as many).  8192 tokens, 128 / 64 tiles, us: n = 1024 bf16 143 / 96,
-  // fp32 460 / 195; 2304 (171 tiles) 152 / 132, 462 / 366; 2816 (253 tiles) 160 / 167, 478 / 521;
-  // 4096 271 / 369, 1092 / 1058; 8192 935 / 1337, 3365 / 4233.
+  // there 64 x 64 tiles (four times as many).  8192 tokens, 128 / 64 tiles, us: n = 1024 bf16 171 / 113,
+  // fp32 482 / 208; 2304 (171 tiles) 175 / 153, 488 / 395; 2432 (190) 172 / 148, 478 / 396; 2560 (210) 176 / 173,
+  // 475 / 521; 2816 (253) 169 / 176, 481 / 532; 4096 286 / 361, 1105 / 1099; 8192 913 / 1322, 3453 / 4145.
   // Up to 256 tokens the time is that of reading and writing H, and smaller tiles spread it over more
   // work-groups: 32 tokens, 128 / 64 tiles, us: 2560 bf16 43 / 30, fp32 43 / 39; 4096 55 / 42, 71 / 57; 8192
   // 133 / 100, 158 / 153; 256 tokens: 2560 47 / 34, 56 / 51; 3584 53 / 45, 66 / 67; 8192 166 / 130, 242 / 226.  At
